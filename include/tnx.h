@@ -73,26 +73,30 @@ int tnx_gemm(int M, int N, int K, int batch, double alpha, const void* A, int a_
              int64_t ldb, int64_t strideB, int b_ncontig, double beta, void* C, int c_f32,
              int64_t ldc, int64_t strideC, int precision, tnx_stream_t stream);
 
-/* GEMM tile choice. Every GEMM takes its tile configuration from the tile
- * table (shape -> configuration) when the shape is there, else from a fixed
- * heuristic; neither allocates, synchronises or changes results (only
- * split-K changes the summation order, and it follows a fixed rule on the
- * shape). The library's only global state is this table, guarded by a
- * mutex.
+/* GEMM tile choice. FP64 and FP32 GEMMs take their tile configuration from a
+ * fixed rule on the shape and the operand types. A BF16X3 GEMM takes it from
+ * the tile table (shape -> configuration) when the shape is there, else from
+ * a fixed heuristic. None of these allocates or synchronises, and the table
+ * does not change results (only sums over parts of K change the summation
+ * order, and they follow the fixed rules). The library's only global state
+ * is this table, guarded by a mutex.
  * tnx_set_autotune(1) turns on an inline tuning mode for tuning runs (off by
  * default; TNX_AUTOTUNE=1 in the environment also turns it on): the first
- * GEMM of a shape missing from the table then times every configuration on a
- * scratch output it allocates with hipMalloc, waits on the stream, and adds
- * the fastest to the table. Mode 1 tunes shapes of at least 2^28
- * multiply-adds; tnx_set_autotune(2) (TNX_AUTOTUNE=2) tunes every shape. Do not use it under graph capture or where the
- * caller cannot allow allocation. tnx_tune_clear empties the table.
+ * BF16X3 GEMM of a shape missing from the table then times every
+ * configuration on a scratch output it allocates with hipMalloc, waits on the
+ * stream, and adds the fastest to the table. Mode 1 tunes shapes of at least
+ * 2^28 multiply-adds; tnx_set_autotune(2) (TNX_AUTOTUNE=2) tunes every shape.
+ * Do not use it under graph capture or where the caller cannot allow
+ * allocation. tnx_tune_clear empties the table.
  * No reference counterpart (quimb leaves this to BLAS). */
 int tnx_set_autotune(int on);
 int tnx_tune_clear(void);
 
 /* Tile table files: tnx_tune_save writes the table to a text file;
  * tnx_tune_load adds a saved table (returns the number of entries, or a
- * negative status). TNX_TUNE_CACHE=<file> in the environment loads a table
+ * negative status; lines of FP64 and FP32 shapes, from tables saved when
+ * those had tiles to choose, are kept and written back, and nothing looks
+ * them up). TNX_TUNE_CACHE=<file> in the environment loads a table
  * before the first GEMM. tnpy_amd loads its committed MI355X table
  * (tnpy_amd/gemm_tiles_mi355x.txt) when it loads the library. No reference
  * counterpart. */

@@ -17,8 +17,8 @@ import numpy as np
 import torch
 
 LIB_PATH = Path(__file__).resolve().parent / "libtnx.so"
-# GEMM tile table chosen by the autotuner on MI355X for the shapes of the
-# DMRG path; loaded with the library so no GEMM is timed inline
+# GEMM tile table chosen by the autotuner on MI355X for the BF16X3 shapes of
+# the DMRG path; loaded with the library so no GEMM is timed inline
 TILE_TABLE = Path(__file__).resolve().parent / "gemm_tiles_mi355x.txt"
 
 TNX_F64, TNX_F32, TNX_BF16X3 = 0, 1, 2

@@ -1,10 +1,11 @@
 // Strided, batched GEMM on CDNA4 matrix cores, the contraction engine of
 // every tensor operation in the library (H_eff matvec stages, environment
-// updates, QR trailing updates, gauge absorption): host side. The kernel
-// template and tile configurations are in gemm_kernel.h; this file holds the
-// split-K rule, the choice between typed and generic staging, the autotuner
-// and the tile table.
-#include "gemm_kernel.h"
+// updates, QR trailing updates, gauge absorption): host side. FP64 and FP32
+// run the kernels of gemm_direct.h, BF16X3 (and what those do not take) the
+// LDS-tile kernels of gemm_kernel.h; this file holds that choice and, for
+// BF16X3, the split-K rule, the choice between typed and generic staging,
+// the autotuner and the tile table.
+#include "gemm_direct.h"
 
 #include <cmath>
 #include <cstdio>
@@ -60,14 +61,6 @@ __global__ void splitk_reduce_kernel(const double* __restrict__ P, int splits, i
 // bitwise identical whichever config runs). Split-K does change the rounding
 // and is therefore decided by a fixed rule on the shape, never by timing.
 // ---------------------------------------------------------------------------
-template <int PREC>
-static void launch_index(int ci, const GemmDesc& d, const GemmArgs& g, int splits, bool typed,
-                         hipStream_t s) {
-  if (PREC == 0) gemm_launch_f64(ci, d, g, splits, typed, s);
-  else if (PREC == 1) gemm_launch_f32(ci, d, g, splits, typed, s);
-  else gemm_launch_bf16(ci, d, g, splits, typed, s);
-}
-
 // One operand of the typed staging: contiguous extent `ext` (elements),
 // leading dimension, batch strides and base all in whole 16-byte vectors,
 // one batch entry (rows x ld, contiguous extent on the last row) < 2 GiB.
@@ -119,12 +112,11 @@ static int split_rule(const GemmDesc& d) {
 
 // Heuristic when not autotuning: fewest full-chip waves, weighted by the
 // per-CU efficiency of the tile size (larger tiles reuse operands more).
-template <int PREC>
 static int heuristic_cfg(const GemmDesc& d, int splits) {
   int best = 0;
   double best_t = 1e300;
-  for (int i = 0; i < Cfgs<PREC>::n; ++i) {
-    const Cfg& c = Cfgs<PREC>::c[i];
+  for (int i = 0; i < Cfgs<2>::n; ++i) {
+    const Cfg& c = Cfgs<2>::c[i];
     const int64_t blocks = (int64_t)ceil_div(d.M, c.bm) * ceil_div(d.N, c.bn) * d.batch * splits;
     const int per_cu = (c.wgm * c.wgn <= 4) ? 2 : 1;
     const double waves = std::ceil((double)blocks / (256.0 * per_cu));
@@ -201,8 +193,9 @@ static int tune_load_locked(const char* path) {
     if (sscanf(line, "%d %d %d %d %d %d %d %d %d %d %d %d", &k.prec, &k.M, &k.N, &k.K, &k.batch,
                &k.ak, &k.bn, &k.ta, &k.tb, &k.tc, &k.splits, &cfg) != 12)
       continue;
-    const int ncfg = k.prec == 0 ? Cfgs<0>::n : (k.prec == 1 ? Cfgs<1>::n : Cfgs<2>::n);
-    if (k.prec < 0 || k.prec > 2 || cfg < 0 || cfg >= ncfg) continue;
+    // lines of the other arithmetics (tables saved when those had tiles to
+    // choose) are kept and written back, but nothing looks them up
+    if (k.prec < 0 || k.prec > 2 || cfg < 0 || cfg >= Cfgs<2>::n) continue;
     g_tune[k] = cfg;
     ++n;
   }
@@ -210,8 +203,7 @@ static int tune_load_locked(const char* path) {
   return n;
 }
 
-template <int PREC>
-static int run_prec(const GemmDesc& d, hipStream_t s) {
+static GemmArgs args_of(const GemmDesc& d) {
   GemmArgs g;
   g.M = d.M; g.N = d.N; g.K = d.K;
   g.A = d.A; g.lda = d.lda; g.sA = d.sA; g.ta = (int)d.ta;
@@ -223,16 +215,54 @@ static int run_prec(const GemmDesc& d, hipStream_t s) {
   g.nb2 = d.nb2 > 0 ? d.nb2 : 1;
   g.sA2 = d.sA2; g.sB2 = d.sB2; g.sC2 = d.sC2;
   g.bidx = d.bidx;
-  const int splits = split_rule(d);
   g.kc = d.K;
   g.partial = nullptr;
+  return g;
+}
+
+// One operand of the direct kernels: a pair to load along its contiguous
+// dimension (extent >= 2), and the offsets of a wave's tile (at most 128
+// rows of a K-contiguous operand, 8 k's of the others, and the contiguous
+// extent of the tile) within the 2 GiB range of a buffer.
+static bool direct_operand_ok(DT t, int64_t ld, int64_t ext, bool kcontig) {
+  const int64_t es = t == DT::F64 ? 8 : 4, lim = ((int64_t)1 << 31) - 4096;
+  return ext >= 2 && (kcontig ? 128 : 8) * std::abs(ld) * es < lim;
+}
+
+bool gemm_direct_ok(const GemmDesc& d) {
+  if (d.prec == Prec::BF16X3 || (d.prec == Prec::F64 && d.ta != DT::F64)) return false;
+  return d.K >= 1 && d.lda >= 0 && d.ldb >= 0 &&
+         direct_operand_ok(d.ta, d.lda, d.a_kcontig ? d.K : d.M, d.a_kcontig) &&
+         direct_operand_ok(d.tb, d.ldb, d.b_ncontig ? d.N : d.K, !d.b_ncontig);
+}
+
+// FP64 and FP32. The configuration follows a fixed rule on the shape and
+// the operand types (never on timing, addresses or strides), since the
+// K-part sum changes the rounding.
+static int run_direct(const GemmDesc& d, hipStream_t s) {
+  const GemmArgs g = args_of(d);
+  const bool f64 = d.prec == Prec::F64;
+  if (gemm_direct_ok(d)) {
+    if (f64) gemm_direct_f64(d, g, s);
+    else gemm_direct_f32(d, g, s);
+  } else {
+    if (f64) gemm_launch_f64(d, g, s);
+    else gemm_launch_f32(d, g, s);
+  }
+  TNX_LAUNCH_CHECK();
+  return TNX_OK;
+}
+
+static int run_bf16(const GemmDesc& d, hipStream_t s) {
+  GemmArgs g = args_of(d);
+  const int splits = split_rule(d);
   if (splits > 1) {
     g.kc = ((d.K + splits - 1) / splits + 31) / 32 * 32;
     g.partial = d.splitk_ws;
   }
   const int nsplit = splits > 1 ? ceil_div(d.K, g.kc) : 1;
   const bool typed = gemm_typed_ok(d, g.kc);
-  const TuneKey key{PREC, d.M, d.N, d.K, d.batch, d.a_kcontig, d.b_ncontig, (int)d.ta, (int)d.tb,
+  const TuneKey key{2, d.M, d.N, d.K, d.batch, d.a_kcontig, d.b_ncontig, (int)d.ta, (int)d.tb,
                     (int)d.tc, nsplit};
   int ci = -1;
   {
@@ -241,7 +271,7 @@ static int run_prec(const GemmDesc& d, hipStream_t s) {
     if (it != g_tune.end()) ci = it->second;
   }
   if (ci < 0) {
-    ci = heuristic_cfg<PREC>(d, nsplit);
+    ci = heuristic_cfg(d, nsplit);
     const int64_t work = (int64_t)d.M * d.N * d.K * d.batch;
     // mode 1 tunes shapes of at least 2^28 multiply-adds, mode 2 every shape
     const int64_t min_work = g_autotune.load() >= 2 ? 0 : ((int64_t)1 << 28);
@@ -265,12 +295,12 @@ static int run_prec(const GemmDesc& d, hipStream_t s) {
           float best = 1e30f;
           int pick = ci;
           bool ok = true;
-          for (int i = 0; ok && i < Cfgs<PREC>::n; ++i) {
-            launch_index<PREC>(i, d, gt, nsplit, typed, s);  // warm
+          for (int i = 0; ok && i < Cfgs<2>::n; ++i) {
+            gemm_launch_bf16(i, d, gt, nsplit, typed, s);  // warm
             float ms = 0.f;
             ok = hipEventRecord(e0, s) == hipSuccess;
-            launch_index<PREC>(i, d, gt, nsplit, typed, s);
-            launch_index<PREC>(i, d, gt, nsplit, typed, s);
+            gemm_launch_bf16(i, d, gt, nsplit, typed, s);
+            gemm_launch_bf16(i, d, gt, nsplit, typed, s);
             ok = ok && hipEventRecord(e1, s) == hipSuccess &&
                  hipEventSynchronize(e1) == hipSuccess &&
                  hipEventElapsedTime(&ms, e0, e1) == hipSuccess;
@@ -288,7 +318,7 @@ static int run_prec(const GemmDesc& d, hipStream_t s) {
     std::lock_guard<std::mutex> lk(g_tune_mu);
     g_tune[key] = ci;
   }
-  launch_index<PREC>(ci, d, g, nsplit, typed, s);
+  gemm_launch_bf16(ci, d, g, nsplit, typed, s);
   TNX_LAUNCH_CHECK();
   if (g.partial) {
     const int64_t MN = (int64_t)d.M * d.N;
@@ -307,9 +337,9 @@ int gemm(const GemmDesc& d, hipStream_t s) {
   TNX_CHECK_ARG(d.A && d.B && d.C, "gemm: null operand");
   TNX_CHECK_ARG(d.batch <= 65535, "gemm: batch %d exceeds 65535", d.batch);
   switch (d.prec) {
-    case Prec::F64: return run_prec<0>(d, s);
-    case Prec::F32: return run_prec<1>(d, s);
-    case Prec::BF16X3: return run_prec<2>(d, s);
+    case Prec::F64:
+    case Prec::F32: return run_direct(d, s);
+    case Prec::BF16X3: return run_bf16(d, s);
   }
   set_error("gemm: unknown precision");
   return TNX_ERR_INVALID;

@@ -1,14 +1,16 @@
-// Kernel instantiations and launcher of the GEMM in arithmetic F64 (FP64 MFMA).
-#include "gemm_kernel.h"
+// Kernel instantiations and launchers of the GEMM in arithmetic F64 (FP64 MFMA).
+#include "gemm_direct.h"
 
 namespace tnx {
 
-void gemm_launch_f64(int ci, const GemmDesc& d, const GemmArgs& g, int splits, bool typed,
-                    hipStream_t s) {
-  if (!typed) return gemm_launch_index<0, void, void>(ci, d, g, splits, s);
-  if (d.ta == DT::F64 && d.tb == DT::F64) return gemm_launch_index<0, double, double>(ci, d, g, splits, s);
-  // (F64, F32): the only other pair gemm_typed_ok admits for F64
-  return gemm_launch_index<0, double, float>(ci, d, g, splits, s);
+void gemm_direct_f64(const GemmDesc& d, const GemmArgs& g, hipStream_t s) {
+  // (F64, F64) and (F64, F32): the pairs gemm_direct_ok admits for F64
+  if (d.tb == DT::F64) return gemm_direct_run<0, double, double>(d, g, s);
+  return gemm_direct_run<0, double, float>(d, g, s);
+}
+
+void gemm_launch_f64(const GemmDesc& d, const GemmArgs& g, hipStream_t s) {
+  gemm_launch_index<0, void, void>(0, d, g, 1, s);
 }
 
 }  // namespace tnx

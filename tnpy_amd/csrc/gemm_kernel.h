@@ -1,8 +1,11 @@
-// Strided, batched GEMM on CDNA4 matrix cores: the kernel template, its tile
-// configurations and the per-configuration launchers. The host side (split-K
-// rule, autotuner, tile table) is in gemm.hip; each arithmetic's kernels are
-// instantiated in a file of their own (gemm_f64.hip, gemm_f32.hip,
-// gemm_bf16.hip) so the three compile in parallel.
+// Strided, batched GEMM on CDNA4 matrix cores through LDS tiles: the kernel
+// template, its tile configurations and the per-configuration launchers. The
+// host side (split-K rule, autotuner, tile table) is in gemm.hip. This form
+// runs the BF16X3 arithmetic, whose operands are split into two bf16 planes
+// once per tile, and the FP64 / FP32 products that gemm_direct.h (registers
+// straight from memory, faster everywhere else) does not take: operands
+// without a pair along their contiguous dimension, or mixed types it has no
+// instantiation for.
 //
 // One kernel template, three arithmetics:
 //   F64    : v_mfma_f64_16x16x4_f64, FP64 LDS tiles [BK][BM]
@@ -13,16 +16,16 @@
 //            8 consecutive k values with one 16-byte LDS read.
 // Tile configurations (block tile BM x BN, WGM x WGN wavefronts of 64 lanes,
 // K-tile depth BK) are listed in Cfgs below; the autotuner picks one per
-// shape. Each wave owns a (BM/WGM) x (BN/WGN) sub-tile of 16x16 MFMA
+// BF16X3 shape. Each wave owns a (BM/WGM) x (BN/WGN) sub-tile of 16x16 MFMA
 // accumulators. Global loads of tile t+1 are issued before the MFMAs of tile
 // t and their results are first used after them; LDS is double-buffered (one
 // barrier per k-tile).
 //
 // Two ways to stage a tile from HBM into LDS, chosen per launch:
-//   * typed (TA, TB = double or float, fixed at compile time): 16-byte
-//     buffer loads along each operand's contiguous dimension. Every vector's
-//     byte offset is computed once, before the k loop; the k step is a
-//     scalar offset. Vectors outside the matrix get an offset beyond the
+//   * typed (BF16X3; TA, TB = double or float, fixed at compile time):
+//     16-byte buffer loads along each operand's contiguous dimension. Every
+//     vector's byte offset is computed once, before the k loop; the k step is
+//     a scalar offset. Vectors outside the matrix get an offset beyond the
 //     buffer's range, which the hardware turns into zeros, so the loop has
 //     no bounds branches. Needs the contiguous extent, the leading dimension
 //     and the base addresses in whole 16-byte vectors, and one batch entry
@@ -62,6 +65,26 @@ struct GemmArgs {
   const int* bidx;  // launched -> logical batch index, or null
 };
 
+// The output tile of this workgroup.
+__device__ __forceinline__ int gemm_tile_of(const GemmArgs& g) {
+  if (g.group_m <= 0) return blockIdx.x;
+  // XCD-aware tile order. Consecutive workgroups are dispatched to the 8
+  // XCDs in turn, each XCD with its own L2: workgroup x takes place x / 8
+  // of a contiguous range of tile ids kept for XCD x % 8. Tile ids run
+  // through groups of group_m tile rows, column by column inside a group,
+  // so an XCD's range is a compact block of tiles that share A row panels
+  // and B column panels in its L2. A bijection on [0, gridDim.x) for any
+  // grid size; each tile is computed exactly as in row-major order.
+  const int T = gridDim.x, x = blockIdx.x & 7, per = T >> 3, rem = T & 7;
+  const int lin = x * per + min(x, rem) + (blockIdx.x >> 3);
+  const int gw = g.group_m * g.tiles_n;
+  const int grp = lin / gw;
+  const int fm = grp * g.group_m;
+  const int gs = min(T / g.tiles_n - fm, g.group_m);
+  const int w = lin - grp * gw;
+  return (fm + w % gs) * g.tiles_n + w / gs;
+}
+
 template <int PREC> struct PT;
 template <> struct PT<0> { using lds_t = double; using acc_t = f64x4; };
 template <> struct PT<1> { using lds_t = float;  using acc_t = f32x4; };
@@ -95,6 +118,7 @@ __global__ __launch_bounds__(64 * WGM * WGN) void gemm_kernel(GemmArgs g) {
   using lds_t = typename PT<PREC>::lds_t;
   using acc_t = typename PT<PREC>::acc_t;
   constexpr bool TYPED = !std::is_void<TA>::value;
+  static_assert(!TYPED || PREC == 2, "typed staging: BF16X3 only");
   constexpr int NT = 64 * WGM * WGN;
   constexpr int EA = BM * BK / NT;
   constexpr int EB = BK * BN / NT;
@@ -119,24 +143,7 @@ __global__ __launch_bounds__(64 * WGM * WGN) void gemm_kernel(GemmArgs g) {
   const int wn0 = (wave % WGN) * WN;
 
   const int bat = g.bidx ? g.bidx[blockIdx.y] : (int)blockIdx.y;
-  int tile = blockIdx.x;
-  if (g.group_m > 0) {
-    // XCD-aware tile order. Consecutive workgroups are dispatched to the 8
-    // XCDs in turn, each XCD with its own L2: workgroup x takes place x / 8
-    // of a contiguous range of tile ids kept for XCD x % 8. Tile ids run
-    // through groups of group_m tile rows, column by column inside a group,
-    // so an XCD's range is a compact block of tiles that share A row panels
-    // and B column panels in its L2. A bijection on [0, gridDim.x) for any
-    // grid size; each tile is computed exactly as in row-major order.
-    const int T = gridDim.x, x = blockIdx.x & 7, per = T >> 3, rem = T & 7;
-    const int lin = x * per + min(x, rem) + (blockIdx.x >> 3);
-    const int gw = g.group_m * g.tiles_n;
-    const int grp = lin / gw;
-    const int fm = grp * g.group_m;
-    const int gs = min(T / g.tiles_n - fm, g.group_m);
-    const int w = lin - grp * gw;
-    tile = (fm + w % gs) * g.tiles_n + w / gs;
-  }
+  const int tile = gemm_tile_of(g);
   const int split = blockIdx.z;
   const int kbeg = split * g.kc;
   const int kend = min(g.K, kbeg + g.kc);
@@ -298,27 +305,11 @@ __global__ __launch_bounds__(64 * WGM * WGN) void gemm_kernel(GemmArgs g) {
         if (!live_a(e)) continue;
         int mi, ki;
         vec_a(e, mi, ki);
-        if constexpr (PREC != 2 && !A_K) {
-          // VA consecutive m of one k row: one vector LDS store
-          lds_t* p = &As[buf][ki * (BM + PADM) + mi];
-          if constexpr (PREC == 0 && VA == 2) {
-            *reinterpret_cast<f64x2*>(p) = f64x2{(double)vec_elem<TA>(va[e], 0), (double)vec_elem<TA>(va[e], 1)};
-          } else if constexpr (PREC == 1 && VA == 2) {
-            *reinterpret_cast<f32x2*>(p) = f32x2{(float)vec_elem<TA>(va[e], 0), (float)vec_elem<TA>(va[e], 1)};
-          } else if constexpr (PREC == 1 && VA == 4) {
-            *reinterpret_cast<f32x4*>(p) = f32x4{vec_elem<float>(va[e], 0), vec_elem<float>(va[e], 1),
-                                                 vec_elem<float>(va[e], 2), vec_elem<float>(va[e], 3)};
-          } else {
 #pragma unroll
-            for (int j = 0; j < VA; ++j) p[j] = (lds_t)vec_elem<TA>(va[e], j);
-          }
-        } else {
-#pragma unroll
-          for (int j = 0; j < VA; ++j) {
-            const TA x = vec_elem<TA>(va[e], j);
-            if (A_K) put_a(buf, mi, ki + j, (float)x, (double)x);
-            else put_a(buf, mi + j, ki, (float)x, (double)x);
-          }
+        for (int j = 0; j < VA; ++j) {
+          const TA x = vec_elem<TA>(va[e], j);
+          if (A_K) put_a(buf, mi, ki + j, (float)x, (double)x);
+          else put_a(buf, mi + j, ki, (float)x, (double)x);
         }
       }
 #pragma unroll
@@ -326,26 +317,11 @@ __global__ __launch_bounds__(64 * WGM * WGN) void gemm_kernel(GemmArgs g) {
         if (!live_b(e)) continue;
         int ni, ki;
         vec_b(e, ni, ki);
-        if constexpr (PREC != 2 && B_N) {
-          lds_t* p = &Bs[buf][ki * (BN + PADM) + ni];
-          if constexpr (PREC == 0 && VB == 2) {
-            *reinterpret_cast<f64x2*>(p) = f64x2{(double)vec_elem<TB>(vb[e], 0), (double)vec_elem<TB>(vb[e], 1)};
-          } else if constexpr (PREC == 1 && VB == 2) {
-            *reinterpret_cast<f32x2*>(p) = f32x2{(float)vec_elem<TB>(vb[e], 0), (float)vec_elem<TB>(vb[e], 1)};
-          } else if constexpr (PREC == 1 && VB == 4) {
-            *reinterpret_cast<f32x4*>(p) = f32x4{vec_elem<float>(vb[e], 0), vec_elem<float>(vb[e], 1),
-                                                 vec_elem<float>(vb[e], 2), vec_elem<float>(vb[e], 3)};
-          } else {
 #pragma unroll
-            for (int j = 0; j < VB; ++j) p[j] = (lds_t)vec_elem<TB>(vb[e], j);
-          }
-        } else {
-#pragma unroll
-          for (int j = 0; j < VB; ++j) {
-            const TB x = vec_elem<TB>(vb[e], j);
-            if (B_N) put_b(buf, ni + j, ki, (float)x, (double)x);
-            else put_b(buf, ni, ki + j, (float)x, (double)x);
-          }
+        for (int j = 0; j < VB; ++j) {
+          const TB x = vec_elem<TB>(vb[e], j);
+          if (B_N) put_b(buf, ni + j, ki, (float)x, (double)x);
+          else put_b(buf, ni, ki + j, (float)x, (double)x);
         }
       }
     } else {
@@ -386,24 +362,6 @@ __global__ __launch_bounds__(64 * WGM * WGN) void gemm_kernel(GemmArgs g) {
     return g.tc == 0 ? reinterpret_cast<const double*>(Cb)[off]
                      : (double)reinterpret_cast<const float*>(Cb)[off];
   };
-  // Small wave tiles (at most 4 accumulator tiles, the 64x64 block) load
-  // their old C values before the first operand tiles, so with beta != 0
-  // the two reads overlap instead of the epilogue waiting for a second
-  // round trip (the rank-32 and rank-128 updates of the blocked QR: one or
-  // a few k-tiles).
-  constexpr bool PRE_C = TM * TN <= 4;
-  const bool pre_c = PRE_C && g.beta != 0.0 && !g.partial;
-  double cpre[PRE_C ? TM : 1][PRE_C ? TN : 1][4];
-  if constexpr (PRE_C) {
-    if (pre_c) {
-#pragma unroll
-      for (int i = 0; i < TM; ++i)
-#pragma unroll
-        for (int j = 0; j < TN; ++j)
-#pragma unroll
-          for (int v = 0; v < 4; ++v) cpre[i][j][v] = load_c(i, j, v);
-    }
-  }
   load_tiles(0);
   store_tiles(0);
   __syncthreads();
@@ -477,9 +435,9 @@ __global__ __launch_bounds__(64 * WGM * WGN) void gemm_kernel(GemmArgs g) {
     return;
   }
   // One 16-row band of the wave's tile at a time: with beta != 0 all of the
-  // band's old C values are loaded first (or were, before the k loop), then
-  // combined and stored (a load placed after the previous element's store
-  // would wait for it, since the compiler cannot tell the addresses apart).
+  // band's old C values are loaded first, then combined and stored (a load
+  // placed after the previous element's store would wait for it, since the
+  // compiler cannot tell the addresses apart).
 #pragma unroll
   for (int i = 0; i < TM; ++i) {
     double cv[TN][4];
@@ -487,13 +445,7 @@ __global__ __launch_bounds__(64 * WGM * WGN) void gemm_kernel(GemmArgs g) {
     for (int j = 0; j < TN; ++j)
 #pragma unroll
       for (int v = 0; v < 4; ++v) {
-        cv[j][v] = 0.0;
-        if constexpr (PRE_C) {
-          if (pre_c) cv[j][v] = cpre[i][j][v];
-          else if (g.beta != 0.0) cv[j][v] = load_c(i, j, v);
-        } else {
-          if (g.beta != 0.0) cv[j][v] = load_c(i, j, v);
-        }
+        cv[j][v] = g.beta != 0.0 ? load_c(i, j, v) : 0.0;
       }
 #pragma unroll
     for (int j = 0; j < TN; ++j)
@@ -519,16 +471,9 @@ __global__ __launch_bounds__(64 * WGM * WGN) void gemm_kernel(GemmArgs g) {
 // ---------------------------------------------------------------------------
 struct Cfg { int bm, bn, wgm, wgn, bk; };
 
-template <int PREC> struct Cfgs;
-template <> struct Cfgs<0> {
-  static constexpr int n = 6;
-  static constexpr Cfg c[n] = {{64, 64, 2, 2, 32}, {128, 128, 2, 2, 32}, {256, 128, 4, 2, 16},
-                               {128, 256, 2, 4, 16}, {256, 160, 4, 2, 16}, {160, 256, 2, 4, 16}};
-};
-template <> struct Cfgs<1> {
-  static constexpr int n = 6;
-  static constexpr Cfg c[n] = {{64, 64, 2, 2, 32}, {128, 128, 2, 2, 32}, {256, 128, 4, 2, 32},
-                               {128, 256, 2, 4, 32}, {256, 160, 4, 2, 32}, {160, 256, 2, 4, 32}};
+template <int PREC> struct Cfgs {  // FP64 and FP32: what gemm_direct.h does not take
+  static constexpr int n = 1;
+  static constexpr Cfg c[n] = {{64, 64, 2, 2, 32}};
 };
 template <> struct Cfgs<2> {
   static constexpr int n = 6;
@@ -536,11 +481,12 @@ template <> struct Cfgs<2> {
                                {128, 256, 2, 4, 32}, {256, 160, 4, 2, 32}, {160, 256, 2, 4, 32}};
 };
 
-// Launch of config `ci` of arithmetic PREC. `typed` selects the typed
-// staging (the caller has checked gemm_typed_ok); defined per arithmetic in
-// gemm_f64.hip, gemm_f32.hip and gemm_bf16.hip.
-void gemm_launch_f64(int ci, const GemmDesc& d, const GemmArgs& g, int splits, bool typed, hipStream_t s);
-void gemm_launch_f32(int ci, const GemmDesc& d, const GemmArgs& g, int splits, bool typed, hipStream_t s);
+// Launches per arithmetic (gemm_f64.hip, gemm_f32.hip, gemm_bf16.hip).
+// gemm_launch_f64 / _f32: the generic form of FP64 / FP32. gemm_launch_bf16:
+// config `ci`; `typed` selects the typed staging (the caller has checked
+// gemm_typed_ok).
+void gemm_launch_f64(const GemmDesc& d, const GemmArgs& g, hipStream_t s);
+void gemm_launch_f32(const GemmDesc& d, const GemmArgs& g, hipStream_t s);
 void gemm_launch_bf16(int ci, const GemmDesc& d, const GemmArgs& g, int splits, bool typed, hipStream_t s);
 
 // True when the typed staging applies: the operand types are an
