@@ -15,9 +15,11 @@
 //     T2[a,w,c,s] = sum_k,v W[w,v,k,c] T1[a,k,v,s]        W-apply
 //     R'[a,w,b]   = sum_c,s T2[a,w,c,s] A[b,c,s]          GEMM (B k-contiguous)
 // The GEMMs carry 2*D*d*chi^3 flops each; the W-apply is a D*d-wide local
-// map, bound by HBM (each (outer, inner) pair reads d*Dr values and writes
-// Dl*d values, coalesced along the inner bond index).
+// map on the matrix cores, bound by HBM (each (outer, inner) pair reads d*Dr
+// values and writes Dl*d values, coalesced along the inner bond index).
 #include "tnx_common.h"
+
+#include <type_traits>
 
 namespace tnx {
 
@@ -27,7 +29,7 @@ namespace tnx {
 //   mode 1 (left env)          : p=v, q=c, x=w, y=k : C = W[w][v][k][c]
 struct WApply {
   const void* in; void* out; const double* W;
-  int in_f32, out_f32;
+  int in_f32;  // in and out are float (else double)
   int64_t n_outer, n_inner;
   int64_t in_so, in_sx, in_sy;     // strides of o, x, y in `in`
   int64_t out_so, out_sp, out_sq;  // strides of o, p, q in `out`
@@ -39,65 +41,135 @@ struct WApply {
   const int* bidx = nullptr;  // launched -> logical problem, or null
 };
 
-template <int MAXIN>
+// The local map on the FP64 matrix cores: out = C in, C (outputs x inputs,
+// at most 64 x 64) in registers as the A operand, the inputs of 32 points as
+// the B operand. A matrix of D d rows per point is far below the matrix
+// cores' rate, so the kernel is left bound by HBM (each value read and
+// written once) or, at small bonds, by one round of loads. The form before
+// (one point per thread, C in LDS, D d dot products of D d terms each on the
+// VALU) measured 51 us at chi = 1024, D = 5 (168 MB), 12 us at chi = 32 and
+// 137 us at chi = 200 with D = 25; this one 27 (6.1 TB/s), 3.9 and 20 us.
+//
+// A wave takes 16 pairs of neighbouring points at a time: lane (i = lane %
+// 16, g = lane / 16) loads input rows t = 4 ks + g of pair i (two points,
+// one 16-byte load of doubles) and feeds the pair's points to two MFMA
+// columns, so an output row is stored as pairs too. Pairs lie along the
+// inner index and are numbered through all outer ones, so short inner
+// extents still fill the wave; the last pair of an odd extent is loaded one
+// point back. PAIR = false (inner extent 1): one point per lane. Inputs past
+// the last row are zero and never loaded from outside.
+typedef double wa_f64x2 __attribute__((ext_vector_type(2), aligned(8)));
+typedef float wa_f32x2 __attribute__((ext_vector_type(2), aligned(4)));
+typedef double wa_f64x4 __attribute__((ext_vector_type(4)));
+
+template <int KS, bool PAIR, typename T>
 __global__ __launch_bounds__(256) void wapply_kernel(WApply a) {
-  __shared__ double C[64 * 64];
+  using T2 = typename std::conditional<sizeof(T) == 8, wa_f64x2, wa_f32x2>::type;
   const int nin = a.NX * a.NY, nout = a.NP * a.NQ;
-  {
-    const int b = a.bidx ? a.bidx[blockIdx.y] : (int)blockIdx.y;
-    a.in = (const char*)a.in + (size_t)b * a.in_sb * (a.in_f32 ? 4 : 8);
-    a.out = (char*)a.out + (size_t)b * a.out_sb * (a.out_f32 ? 4 : 8);
-    a.W += (size_t)b * a.W_sb;
-  }
-  for (int t = threadIdx.x; t < nout * nin; t += blockDim.x) {
-    const int oi = t / nin, ii = t % nin;
-    const int p = oi / a.NQ, q = oi % a.NQ;
-    const int x = ii / a.NY, y = ii % a.NY;
-    int w, v, k, c;
-    if (a.mode == 0) { w = p; c = q; k = x; v = y; }
-    else             { v = p; c = q; w = x; k = y; }
-    C[t] = a.W[((w * a.Dr + v) * a.d + k) * a.d + c];
-  }
-  __syncthreads();
-  const int64_t total = a.n_outer * a.n_inner;
-  for (int64_t g = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; g < total;
-       g += (int64_t)gridDim.x * blockDim.x) {
-    const int64_t o = g / a.n_inner, i = g % a.n_inner;
-    double xin[MAXIN];
+  const int lane = threadIdx.x & 63, li = lane & 15, lg = lane >> 4;
+  const int b = a.bidx ? a.bidx[blockIdx.y] : (int)blockIdx.y;
+  const T* in = (const T*)a.in + (int64_t)b * a.in_sb;
+  T* out = (T*)a.out + (int64_t)b * a.out_sb;
+  const double* W = a.W + (int64_t)b * a.W_sb;
+  // C's fragments: row r0 + li, column 4 ks + lg
+  const int r0 = 16 * blockIdx.z;
+  double c[KS];
 #pragma unroll
-    for (int t = 0; t < MAXIN; ++t) {
-      if (t < nin) {
-        const int x = t / a.NY, y = t % a.NY;
-        const int64_t off = o * a.in_so + x * a.in_sx + y * a.in_sy + i;
-        xin[t] = a.in_f32 ? (double)reinterpret_cast<const float*>(a.in)[off]
-                          : reinterpret_cast<const double*>(a.in)[off];
+  for (int ks = 0; ks < KS; ++ks) {
+    const int r = r0 + li, t = 4 * ks + lg;
+    c[ks] = 0.0;
+    if (r < nout && t < nin) {
+      const int p = r / a.NQ, q = r % a.NQ, x = t / a.NY, y = t % a.NY;
+      const int w = a.mode == 0 ? p : x, v = a.mode == 0 ? y : p, k = a.mode == 0 ? x : y;
+      c[ks] = W[((w * a.Dr + v) * a.d + k) * a.d + q];
+    }
+  }
+  int64_t irow[KS];  // offset of input row 4 ks + lg (row 0 past the last)
+#pragma unroll
+  for (int ks = 0; ks < KS; ++ks) {
+    const int t = 4 * ks + lg;
+    irow[ks] = t < nin ? (t / a.NY) * a.in_sx + (t % a.NY) * a.in_sy : 0;
+  }
+  int64_t orow[4];  // offset of output row r0 + lg + 4 v
+#pragma unroll
+  for (int v = 0; v < 4; ++v) {
+    const int r = r0 + lg + 4 * v;
+    orow[v] = (r / a.NQ) * a.out_sp + (r % a.NQ) * a.out_sq;
+  }
+  const unsigned inner = (unsigned)a.n_inner;
+  const unsigned per = PAIR ? (inner + 1) / 2 : inner;  // columns per outer index
+  const int64_t total = (int64_t)a.n_outer * per;
+  const int64_t wave = ((int64_t)blockIdx.x * blockDim.x + threadIdx.x) >> 6;
+  const int64_t waves = ((int64_t)gridDim.x * blockDim.x) >> 6;
+  for (int64_t c0 = wave * 16; c0 < total; c0 += waves * 16) {
+    const int64_t col = c0 + li;
+    const bool on = col < total;
+    const unsigned pc = (unsigned)(on ? col : 0);
+    const unsigned o = pc / per;
+    const unsigned i = (pc - o * per) * (PAIR ? 2 : 1);
+    const bool half = PAIR && i + 1 == inner;  // odd extent: one point left
+    const T* src = in + (int64_t)o * a.in_so + (half ? i - 1 : i);
+    double x0[KS], x1[KS];
+#pragma unroll
+    for (int ks = 0; ks < KS; ++ks) {
+      const bool in_k = 4 * ks + lg < nin;
+      if constexpr (PAIR) {
+        const T2 v = *reinterpret_cast<const T2*>(src + irow[ks]);
+        x0[ks] = in_k ? (double)(half ? v[1] : v[0]) : 0.0;
+        x1[ks] = in_k ? (double)v[1] : 0.0;
+      } else {
+        x0[ks] = in_k ? (double)src[irow[ks]] : 0.0;
       }
     }
-    for (int oi = 0; oi < nout; ++oi) {
-      const int p = oi / a.NQ, q = oi % a.NQ;
-      double s = 0.0;
+    wa_f64x4 y0 = {0.0, 0.0, 0.0, 0.0}, y1 = {0.0, 0.0, 0.0, 0.0};
 #pragma unroll
-      for (int t = 0; t < MAXIN; ++t)
-        if (t < nin) s += C[oi * nin + t] * xin[t];
-      const int64_t off = o * a.out_so + p * a.out_sp + q * a.out_sq + i;
-      if (a.out_f32) reinterpret_cast<float*>(a.out)[off] = (float)s;
-      else reinterpret_cast<double*>(a.out)[off] = s;
+    for (int ks = 0; ks < KS; ++ks) {
+      y0 = __builtin_amdgcn_mfma_f64_16x16x4f64(c[ks], x0[ks], y0, 0, 0, 0);
+      if constexpr (PAIR) y1 = __builtin_amdgcn_mfma_f64_16x16x4f64(c[ks], x1[ks], y1, 0, 0, 0);
+    }
+    // element v sits at row lg + 4 v, column li
+#pragma unroll
+    for (int v = 0; v < 4; ++v) {
+      if (!on || r0 + lg + 4 * v >= nout) continue;
+      T* dst = out + (int64_t)o * a.out_so + orow[v] + i;
+      if (PAIR && !half) *reinterpret_cast<T2*>(dst) = T2{(T)y0[v], (T)y1[v]};
+      else *dst = (T)y0[v];
     }
   }
 }
 
 static int launch_wapply(const WApply& a, hipStream_t s) {
-  const int nin = a.NX * a.NY;
-  TNX_CHECK_ARG(a.NP * a.NQ <= 64 && nin <= 64,
-                "W-apply: D*d = %d / %d exceeds 64", a.NP * a.NQ, nin);
-  const int64_t total = a.n_outer * a.n_inner;
-  if (total == 0) return TNX_OK;
+  const int nin = a.NX * a.NY, nout = a.NP * a.NQ;
+  TNX_CHECK_ARG(nout <= 64 && nin <= 64,
+                "W-apply: D*d = %d / %d exceeds 64", nout, nin);
+  if (a.n_outer * a.n_inner == 0) return TNX_OK;
   TNX_CHECK_ARG(a.batch >= 1 && a.batch <= 65535, "W-apply: bad batch %d", a.batch);
-  int blocks = (int)std::min<int64_t>((total + 255) / 256, std::max<int64_t>(8192 / a.batch, 64));
-  if (nin <= 16)
-    hipLaunchKernelGGL(wapply_kernel<16>, dim3(blocks, a.batch), dim3(256), 0, s, a);
-  else
-    hipLaunchKernelGGL(wapply_kernel<64>, dim3(blocks, a.batch), dim3(256), 0, s, a);
+  const bool pair = a.n_inner >= 2;
+  const int64_t cols = a.n_outer * (pair ? (a.n_inner + 1) / 2 : a.n_inner);
+  TNX_CHECK_ARG(cols < ((int64_t)1 << 31), "W-apply: %lld points per problem", (long long)cols);
+  // one 16-column step per wave up to the 8192 waves that the chip holds;
+  // one-wave blocks while those do not reach every CU
+  const int64_t steps = (cols + 15) / 16;
+  const int row_tiles = (nout + 15) / 16;
+  const int nt = steps * a.batch * row_tiles <= 1024 ? 64 : 256;
+  const int64_t blocks =
+      std::min<int64_t>((steps * 64 + nt - 1) / nt, std::max<int64_t>(2048 / ((int64_t)a.batch * row_tiles), 8));
+  const dim3 grid((int)blocks, a.batch, row_tiles), block(nt);
+  auto go = [&](auto ks, auto pr) {
+    constexpr int KS = decltype(ks)::value;
+    constexpr bool PR = decltype(pr)::value;
+    if (a.in_f32) hipLaunchKernelGGL((wapply_kernel<KS, PR, float>), grid, block, 0, s, a);
+    else hipLaunchKernelGGL((wapply_kernel<KS, PR, double>), grid, block, 0, s, a);
+  };
+  auto pick = [&](auto pr) {
+    if (nin <= 12) go(std::integral_constant<int, 3>{}, pr);  // D = 5, 6
+    else if (nin <= 16) go(std::integral_constant<int, 4>{}, pr);
+    else if (nin <= 32) go(std::integral_constant<int, 8>{}, pr);
+    else if (nin <= 52) go(std::integral_constant<int, 13>{}, pr);  // D = 25
+    else go(std::integral_constant<int, 16>{}, pr);
+  };
+  if (pair) pick(std::true_type{});
+  else pick(std::false_type{});
   TNX_LAUNCH_CHECK();
   return TNX_OK;
 }
@@ -165,7 +237,7 @@ int heff1_matvec_b(const void* L, const double* W, const void* R, const void* x,
   g1.alpha = 1.0; g1.beta = 0.0; g1.prec = (Prec)prec;
   TNX_TRY(gemm(g1, s));
   WApply wa{};
-  wa.in = T1; wa.out = T2; wa.W = W; wa.in_f32 = wa.out_f32 = (prec != TNX_F64);
+  wa.in = T1; wa.out = T2; wa.W = W; wa.in_f32 = (prec != TNX_F64);
   wa.n_outer = chil; wa.n_inner = chir;
   wa.in_so = (int64_t)d * Dr * chir; wa.in_sx = (int64_t)Dr * chir; wa.in_sy = chir;
   wa.out_so = (int64_t)Dl * d * chir; wa.out_sp = (int64_t)d * chir; wa.out_sq = chir;
@@ -232,7 +304,7 @@ int heff2_matvec(const double* L, const double* W1, const double* W2, const doub
   g1.alpha = 1.0; g1.beta = 0.0; g1.prec = (Prec)prec;
   TNX_TRY(gemm(g1, s));
   WApply a2{};  // W2 over (k2, v) -> (u, c2), outer (l,k1), inner r'
-  a2.in = T1; a2.out = T2; a2.W = W2; a2.in_f32 = a2.out_f32 = (prec != TNX_F64);
+  a2.in = T1; a2.out = T2; a2.W = W2; a2.in_f32 = (prec != TNX_F64);
   a2.n_outer = (int64_t)chil * d; a2.n_inner = chir;
   a2.in_so = (int64_t)d * Dr * chir; a2.in_sx = (int64_t)Dr * chir; a2.in_sy = chir;
   a2.out_so = (int64_t)Dm * d * chir; a2.out_sp = (int64_t)d * chir; a2.out_sq = chir;
@@ -240,7 +312,7 @@ int heff2_matvec(const double* L, const double* W1, const double* W2, const doub
   a2.Dl = Dm; a2.Dr = Dr; a2.d = d; a2.mode = 0;
   TNX_TRY(launch_wapply(a2, s));
   WApply a1{};  // W1 over (k1, u) -> (w, c1), outer l, inner (c2, r')
-  a1.in = T2; a1.out = T3; a1.W = W1; a1.in_f32 = a1.out_f32 = (prec != TNX_F64);
+  a1.in = T2; a1.out = T3; a1.W = W1; a1.in_f32 = (prec != TNX_F64);
   a1.n_outer = chil; a1.n_inner = (int64_t)d * chir;
   a1.in_so = (int64_t)d * Dm * d * chir; a1.in_sx = (int64_t)Dm * d * chir; a1.in_sy = (int64_t)d * chir;
   a1.out_so = (int64_t)Dl * d * d * chir; a1.out_sp = (int64_t)d * d * chir; a1.out_sq = (int64_t)d * chir;
@@ -290,7 +362,7 @@ int env_left_b(const double* L, const double* A, const double* W, double* Lout,
   g1.alpha = 1.0; g1.beta = 0.0; g1.prec = (Prec)prec;
   TNX_TRY(gemm(g1, s));
   WApply wa{};
-  wa.in = T1; wa.out = T2; wa.W = W; wa.in_f32 = wa.out_f32 = (prec != TNX_F64);
+  wa.in = T1; wa.out = T2; wa.W = W; wa.in_f32 = (prec != TNX_F64);
   wa.n_outer = chil; wa.n_inner = chir;
   wa.in_so = (int64_t)d * chir; wa.in_sx = nA; wa.in_sy = chir;
   wa.out_so = (int64_t)d * chir; wa.out_sp = nA; wa.out_sq = chir;
@@ -340,7 +412,7 @@ int env_right_b(const double* R, const double* A, const double* W, double* Rout,
   g1.alpha = 1.0; g1.beta = 0.0; g1.prec = (Prec)prec;
   TNX_TRY(gemm(g1, s));
   WApply wa{};
-  wa.in = T1; wa.out = T2; wa.W = W; wa.in_f32 = wa.out_f32 = (prec != TNX_F64);
+  wa.in = T1; wa.out = T2; wa.W = W; wa.in_f32 = (prec != TNX_F64);
   wa.n_outer = chil; wa.n_inner = chir;
   wa.in_so = (int64_t)d * Dr * chir; wa.in_sx = (int64_t)Dr * chir; wa.in_sy = chir;
   wa.out_so = (int64_t)Dl * d * chir; wa.out_sp = (int64_t)d * chir; wa.out_sq = chir;
