@@ -13,6 +13,7 @@
 // panel columns fused with the V^T v Gram entries that build the compact-WY
 // factor T). Trailing updates and the explicit Q are GEMMs on MFMA:
 //   A_trail -= V (T^T (V^T A_trail)),   Q_sub -= V (T (V^T Q_sub)).
+#include "qr_chol.h"
 #include "tnx_common.h"
 
 #include <algorithm>
@@ -1339,6 +1340,243 @@ static int launch_panel(const QrCfg& c, double* A, int m, int n, int jb, int b, 
   return TNX_ERR_UNSUPPORTED;
 }
 
+// ---- QR in LDS -----------------------------------------------------------------
+// Householder QR of `batch` small m x n matrices (m >= n), one workgroup per
+// matrix held in LDS (row stride n + 1). trans = 0: matrix p is A_p, m x n
+// row-major. trans = 1: matrix p is A_p^T, where A_p is n x m row-major (the
+// leftward gauge move: A = (Q R)^T). On exit A_p holds the thin Q (Q^T when
+// trans) and R_p = R (n x n, upper triangular). Same reflector convention as
+// the blocked path (beta = -sign(alpha) |x|).
+constexpr int kQrSmallBig = 16640;   // m * (n + 1) doubles: 130 KiB of LDS
+
+// Householder QR of the matrix at A (trans as above) by the whole workgroup
+// in the LDS buffer S (m (n + 1) + 2 n + 16 doubles).
+template <int NT>
+__device__ void qr_lds_householder(double* __restrict__ A, int m, int n, int trans, double* __restrict__ R,
+                                   double* S) {
+  constexpr int NW = NT / 64;
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  const int ld = n + 1, mn = m * n;
+  double* tau_s = S + m * ld;
+  double* sgn = tau_s + n;
+  double* red = sgn + n;
+  for (int e = tid; e < mn; e += NT) {
+    int i, c;
+    if (trans) { c = e / m; i = e - c * m; } else { i = e / n; c = e - i * n; }
+    S[i * ld + c] = A[e];
+  }
+  __syncthreads();
+  lds_householder<NT>(S, ld, m, n, tau_s, red);
+  // ---- R, with a non-negative diagonal (same convention as the blocked QR)
+  for (int j = tid; j < n; j += NT) sgn[j] = S[j * ld + j] < 0.0 ? -1.0 : 1.0;
+  __syncthreads();
+  for (int e = tid; e < n * n; e += NT) {
+    const int i = e / n, c = e - i * n;
+    R[e] = (c >= i) ? sgn[i] * S[i * ld + c] : 0.0;
+  }
+  __syncthreads();
+  // ---- thin Q = H_0 ... H_{n-1} [I; 0], formed in place from the last column
+  for (int j = n - 1; j >= 0; --j) {
+    const double tj = tau_s[j];
+    if (tj != 0.0) {
+      for (int c = j + 1 + wave; c < n; c += NW) {
+        double acc = 0.0;
+        for (int i = j + lane; i < m; i += 64) acc += (i == j ? 1.0 : S[i * ld + j]) * S[i * ld + c];
+        const double w = tj * wsum(acc);
+        for (int i = j + lane; i < m; i += 64) S[i * ld + c] -= (i == j ? 1.0 : S[i * ld + j]) * w;
+      }
+    }
+    __syncthreads();
+    for (int i = tid; i < m; i += NT)
+      S[i * ld + j] = (i < j) ? 0.0 : (i == j ? 1.0 - tj : -tj * S[i * ld + j]);
+    __syncthreads();
+  }
+  for (int e = tid; e < mn; e += NT) {
+    int i, c;
+    if (trans) { c = e / m; i = e - c * m; } else { i = e / n; c = e - i * n; }
+    A[e] = sgn[c] * S[i * ld + c];
+  }
+}
+
+__global__ __launch_bounds__(256) void qr_small_kernel(double* __restrict__ A, int m, int n, int trans,
+                                                       double* __restrict__ R) {
+  __shared__ double S[kQrSmallBig + 2 * 256 + 16];
+  qr_lds_householder<256>(A + (int64_t)blockIdx.x * m * n, m, n, trans, R + (int64_t)blockIdx.x * n * n, S);
+}
+
+// The same factorisation by Cholesky QR (qr_chol.h), where the matrix, its
+// Gram matrix and the diagonal inverses fit in LDS together (up to about
+// 144 x 72): two to four passes of Gram, Cholesky and triangular solve on the
+// matrix cores instead of a chain of 2 n column steps with a block reduction
+// each. A matrix that does not converge (exactly zero columns) or overflows
+// is read again and takes the Householder steps. R's block column w stays in
+// wave w's registers. Bound by the chain of pivots (16 n per pass) and one
+// CU's matrix rate. The gauge move of a 60 x 2 x 60 site, with R times the
+// neighbour: 162 us with two panels of the many-workgroup path, 79 us so; a
+// batch of 64 x 2 x 64 sites took 683 us in the Householder kernel above.
+constexpr int kQcLdsBig = 20200, kQcLdsLittle = 4864;  // 158 and 38 KiB
+
+template <int CAP, int NT, int NB>
+__global__ __launch_bounds__(NT) void qr_chol_kernel(double* __restrict__ A, int m, int n, int trans,
+                                                     double* __restrict__ R) {
+  __shared__ double S[CAP];
+  __shared__ int flag[3];
+  constexpr int NW = NT / 64;
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, lr = lane & 15, lk = lane >> 4;
+  constexpr int nb = NB, ld = 16 * NB + 1;
+  const int mt = (m + 15) / 16;
+  double* G = S + 16 * mt * ld;
+  double* X = G + 16 * nb * ld;
+  double* d0 = X + 16 * nb * kQcXLd;
+  double* Ap = A + (int64_t)blockIdx.x * m * n;
+  double* Rp = R + (int64_t)blockIdx.x * n * n;
+  for (int e = tid; e < 16 * mt * ld; e += NT) S[e] = 0.0;
+  __syncthreads();
+  if (trans) {
+    for (int c = wave; c < n; c += NW)
+#pragma unroll 4
+      for (int i = lane; i < m; i += 64) S[i * ld + c] = Ap[c * m + i];
+  } else {
+#pragma unroll 4
+    for (int i = wave; i < m; i += NW)
+      for (int c = lane; c < n; c += 64) S[i * ld + c] = Ap[i * n + c];
+  }
+  qc_f64x4 Rb[NB];
+  bool done = false;
+  for (int p = 0; p < kQcPasses && !done; ++p) {
+    if (tid < 2) flag[tid] = 0;
+    __syncthreads();
+    // ---- Gram matrix, lower 16 x 16 tiles; identity in the padding
+    bool far = false, bad = false;
+    for (int t = wave; t < nb * (nb + 1) / 2; t += NW) {
+      int bi = 0, bj = t;
+      while (bj > bi) { bj -= bi + 1; ++bi; }
+      const double* Si = S + lk * ld + 16 * bi + lr;
+      const double* Sj = S + lk * ld + 16 * bj + lr;
+      qc_f64x4 g = {0.0, 0.0, 0.0, 0.0}, h = g;
+      for (int k = 0; k < 16 * mt; k += 16) {
+        g = qc_mfma(Si[k * ld], Sj[k * ld], g);
+        h = qc_mfma(Si[(k + 4) * ld], Sj[(k + 4) * ld], h);
+        g = qc_mfma(Si[(k + 8) * ld], Sj[(k + 8) * ld], g);
+        h = qc_mfma(Si[(k + 12) * ld], Sj[(k + 12) * ld], h);
+      }
+#pragma unroll
+      for (int v = 0; v < 4; ++v) {
+        const int i = 16 * bi + lk + 4 * v, c = 16 * bj + lr;
+        double x = g[v] + h[v];
+        if (i == c) {
+          if (i >= n) x = 1.0;
+          d0[i] = x;
+          bad = bad || !(x > 1e-290 && x < 1e290);
+        }
+        if (c <= i) far = far || !(fabs(x - (i == c ? 1.0 : 0.0)) <= 0.1);
+        G[i * ld + c] = x;
+      }
+    }
+    if (far) flag[0] = 1;
+    if (bad) flag[1] = 1;
+    __syncthreads();
+    done = p > 0 && flag[0] == 0;
+    if (flag[1]) break;
+    const bool ill = qc_cholesky<NT, NB, ld>(G, d0, p == 0 ? kQcTau1 : kQcTau2, X, &flag[2]);
+    if (wave < nb) {
+      if (p == 0) {
+#pragma unroll
+        for (int k = 0; k < NB; ++k)
+#pragma unroll
+          for (int v = 0; v < 4; ++v) Rb[k][v] = k <= wave ? G[(16 * wave + lr) * ld + 16 * k + lk + 4 * v] : 0.0;
+      } else {
+        qc_update_r<NB, ld>(Rb, wave, G);
+      }
+    }
+    for (int t = wave; t < mt; t += NW) {
+      double* St = S + (16 * t + lr) * ld + lk;
+      qc_f64x4 Z[NB];
+#pragma unroll
+      for (int j = 0; j < NB; ++j)
+#pragma unroll
+        for (int v = 0; v < 4; ++v) Z[j][v] = St[16 * j + 4 * v];
+      qc_trsm<NB, ld>(Z, G, X, ill);
+#pragma unroll
+      for (int j = 0; j < NB; ++j)
+#pragma unroll
+        for (int v = 0; v < 4; ++v) St[16 * j + 4 * v] = Z[j][v];
+    }
+    __syncthreads();
+  }
+  if (!done) {
+    qr_lds_householder<NT>(Ap, m, n, trans, Rp, S);
+    return;
+  }
+  if (wave < nb) {
+    const int c = 16 * wave + lr;
+#pragma unroll
+    for (int k = 0; k < NB; ++k)
+#pragma unroll
+      for (int v = 0; v < 4; ++v) {
+        const int i = 16 * k + lk + 4 * v;
+        if (i < n && c < n) Rp[i * n + c] = Rb[k][v];
+      }
+  }
+  if (trans) {
+    for (int c = wave; c < n; c += NW)
+#pragma unroll 4
+      for (int i = lane; i < m; i += 64) Ap[c * m + i] = S[i * ld + c];
+  } else {
+#pragma unroll 4
+    for (int i = wave; i < m; i += NW)
+      for (int c = lane; c < n; c += 64) Ap[i * n + c] = S[i * ld + c];
+  }
+}
+
+static int64_t qr_chol_need(int m, int n) {
+  const int64_t m16 = (m + 15) / 16 * 16, n16 = (n + 15) / 16 * 16;
+  return (m16 + n16) * (n16 + 1) + (kQcXLd + 1) * n16;
+}
+
+static bool qr_chol_fits(int m, int n) { return m >= n && n >= 1 && n <= 80 && qr_chol_need(m, n) <= kQcLdsBig; }
+
+static int qr_chol(double* A, int m, int n, int trans, double* R, int batch, hipStream_t s) {
+  const int nb = (n + 15) / 16;
+  // the little form (four waves) leaves room for several matrices on a CU
+  const bool little = nb <= 3 && qr_chol_need(m, n) <= kQcLdsLittle;
+#define TNX_QRC(NB_, CAP_, NT_)                                                                               \
+  case NB_:                                                                                                   \
+    hipLaunchKernelGGL((qr_chol_kernel<CAP_, NT_, NB_>), dim3(batch), dim3(NT_), 0, s, A, m, n, trans, R);    \
+    break;
+  if (little) {
+    switch (nb) {
+      TNX_QRC(1, kQcLdsLittle, 256)
+      TNX_QRC(2, kQcLdsLittle, 256)
+      TNX_QRC(3, kQcLdsLittle, 256)
+    }
+  } else {
+    switch (nb) {
+      TNX_QRC(1, kQcLdsBig, 512)
+      TNX_QRC(2, kQcLdsBig, 512)
+      TNX_QRC(3, kQcLdsBig, 512)
+      TNX_QRC(4, kQcLdsBig, 512)
+      TNX_QRC(5, kQcLdsBig, 512)
+    }
+  }
+#undef TNX_QRC
+  TNX_LAUNCH_CHECK();
+  return TNX_OK;
+}
+
+static bool qr_small_fits(int m, int n) {
+  return m >= n && n >= 1 && n <= 256 && (int64_t)m * (n + 1) <= kQrSmallBig;
+}
+
+static int qr_small_b(double* A, int m, int n, int trans, double* R, int batch, hipStream_t s) {
+  TNX_CHECK_ARG(qr_small_fits(m, n), "qr_batched: %d x %d exceeds the LDS-resident limit", m, n);
+  TNX_CHECK_ARG(batch >= 1 && batch <= 2147483647, "qr_batched: bad batch %d", batch);
+  if (qr_chol_fits(m, n)) return qr_chol(A, m, n, trans, R, batch, s);
+  hipLaunchKernelGGL(qr_small_kernel, dim3(batch), dim3(256), 0, s, A, m, n, trans, R);
+  TNX_LAUNCH_CHECK();
+  return TNX_OK;
+}
+
 // Blocked QR with Cholesky-QR2 panels (three kernels per panel) and two
 // GEMMs per panel for the trailing update; a panel that fails the
 // Cholesky-QR checks sends the whole factorisation to the TSQR panel path
@@ -1584,6 +1822,10 @@ static int qr_tsqr(double* A, int m, int n, double* R, void* ws, hipStream_t s) 
 int qr(double* A, int m, int n, double* R, void* ws, size_t ws_bytes, hipStream_t s) {
   TNX_CHECK_ARG(A && R, "qr: null pointer");
   TNX_CHECK_ARG(m >= 1 && n >= 1 && m >= n, "qr: need m >= n >= 1 (m=%d n=%d)", m, n);
+  if (qr_chol_fits(m, n)) {
+    TNX_CHECK_ARG(ws && ws_bytes >= qr_ws_bytes(m, n), "qr: workspace too small");
+    return qr_chol(A, m, n, 0, R, 1, s);
+  }
   if (ts_fits(m, n)) {
     TNX_CHECK_ARG(ws && ws_bytes >= qr_ws_bytes(m, n), "qr: workspace too small");
     return qr_tsqr(A, m, n, R, ws, s);
@@ -1728,9 +1970,13 @@ int gauge_left(double* A, const double* prev, double* prev_out, int chil, int d,
   double* At = (double*)p; p += al((size_t)m * n * 8);
   double* R = (double*)p; p += al((size_t)n * n * 8);
   // A (chil x d*chir) -> At (d*chir x chil); At = Q R; A = Q^T; prev <- prev R^T
-  TNX_TRY(transpose_f64(A, At, n, m, s));
-  TNX_TRY(qr(At, m, n, R, p, qr_ws_bytes(m, n), s));
-  TNX_TRY(transpose_f64(At, A, m, n, s));
+  if (qr_chol_fits(m, n)) {
+    TNX_TRY(qr_chol(A, m, n, 1, R, 1, s));
+  } else {
+    TNX_TRY(transpose_f64(A, At, n, m, s));
+    TNX_TRY(qr(At, m, n, R, p, qr_ws_bytes(m, n), s));
+    TNX_TRY(transpose_f64(At, A, m, n, s));
+  }
   GemmDesc g{};
   g.M = prev_rows; g.N = n; g.K = n; g.batch = 1;
   g.A = prev; g.ta = DT::F64; g.lda = n; g.sA = 0; g.a_kcontig = true;
@@ -1738,118 +1984,6 @@ int gauge_left(double* A, const double* prev, double* prev_out, int chil, int d,
   g.C = prev_out; g.tc = DT::F64; g.ldc = n; g.sC = 0;
   g.alpha = 1.0; g.beta = 0.0; g.prec = Prec::F64;
   return gemm(g, s);
-}
-
-// ---- batched small QR ----------------------------------------------------------
-// Householder QR of `batch` small m x n matrices (m >= n), one workgroup per
-// matrix held in LDS (row stride n + 1). trans = 0: matrix p is A_p, m x n
-// row-major. trans = 1: matrix p is A_p^T, where A_p is n x m row-major (the
-// leftward gauge move: A = (Q R)^T). On exit A_p holds the thin Q (Q^T when
-// trans) and R_p = R (n x n, upper triangular). Same reflector convention as
-// the blocked path (beta = -sign(alpha) |x|).
-constexpr int kQrSmallBig = 16640;   // m * (n + 1) doubles: 130 KiB of LDS
-constexpr int kQrSmallLittle = 4352; // 34 KiB
-
-__device__ __forceinline__ double qs_block_sum(double v, double* red) {
-  const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
-  v = wsum(v);
-  __syncthreads();
-  if (lane == 0) red[wv] = v;
-  __syncthreads();
-  return (red[0] + red[1]) + (red[2] + red[3]);
-}
-
-template <int MAXE>
-__global__ __launch_bounds__(256) void qr_small_kernel(double* __restrict__ A, int m, int n,
-                                                       int trans, double* __restrict__ R) {
-  __shared__ double S[MAXE];
-  __shared__ double tau_s[256];
-  __shared__ double red[4];
-  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-  const int ld = n + 1;
-  const int64_t mn = (int64_t)m * n;
-  double* Ap = A + (int64_t)blockIdx.x * mn;
-  for (int e = tid; e < mn; e += 256) {
-    int i, c;
-    if (trans) { c = e / m; i = e - c * m; } else { i = e / n; c = e - i * n; }
-    S[i * ld + c] = Ap[e];
-  }
-  __syncthreads();
-  // ---- factorisation
-  for (int j = 0; j < n; ++j) {
-    double part = 0.0;
-    for (int i = j + 1 + tid; i < m; i += 256) part += S[i * ld + j] * S[i * ld + j];
-    const double sigma = qs_block_sum(part, red);
-    const double alpha = S[j * ld + j];
-    double tj = 0.0, beta = alpha, scale = 0.0;
-    if (sigma != 0.0) {
-      const double nrm = sqrt(alpha * alpha + sigma);
-      beta = alpha >= 0.0 ? -nrm : nrm;
-      tj = (beta - alpha) / beta;
-      scale = 1.0 / (alpha - beta);
-    }
-    __syncthreads();
-    for (int i = j + 1 + tid; i < m; i += 256) S[i * ld + j] *= scale;
-    if (tid == 0) { S[j * ld + j] = beta; tau_s[j] = tj; }
-    __syncthreads();
-    if (tj != 0.0) {
-      for (int c = j + 1 + wave; c < n; c += 4) {
-        double acc = 0.0;
-        for (int i = j + lane; i < m; i += 64) acc += (i == j ? 1.0 : S[i * ld + j]) * S[i * ld + c];
-        const double w = tj * wsum(acc);
-        for (int i = j + lane; i < m; i += 64) S[i * ld + c] -= (i == j ? 1.0 : S[i * ld + j]) * w;
-      }
-    }
-    __syncthreads();
-  }
-  // ---- R, with a non-negative diagonal (same convention as the blocked QR)
-  __shared__ double sgn[256];
-  for (int j = tid; j < n; j += 256) sgn[j] = S[j * ld + j] < 0.0 ? -1.0 : 1.0;
-  __syncthreads();
-  double* Rp = R + (int64_t)blockIdx.x * n * n;
-  for (int e = tid; e < n * n; e += 256) {
-    const int i = e / n, c = e - i * n;
-    Rp[e] = (c >= i) ? sgn[i] * S[i * ld + c] : 0.0;
-  }
-  __syncthreads();
-  // ---- thin Q = H_0 ... H_{n-1} [I; 0], formed in place from the last column
-  for (int j = n - 1; j >= 0; --j) {
-    const double tj = tau_s[j];
-    if (tj != 0.0) {
-      for (int c = j + 1 + wave; c < n; c += 4) {
-        double acc = 0.0;
-        for (int i = j + lane; i < m; i += 64) acc += (i == j ? 1.0 : S[i * ld + j]) * S[i * ld + c];
-        const double w = tj * wsum(acc);
-        for (int i = j + lane; i < m; i += 64) S[i * ld + c] -= (i == j ? 1.0 : S[i * ld + j]) * w;
-      }
-    }
-    __syncthreads();
-    for (int i = tid; i < m; i += 256)
-      S[i * ld + j] = (i < j) ? 0.0 : (i == j ? 1.0 - tj : -tj * S[i * ld + j]);
-    __syncthreads();
-  }
-  for (int e = tid; e < mn; e += 256) {
-    int i, c;
-    if (trans) { c = e / m; i = e - c * m; } else { i = e / n; c = e - i * n; }
-    Ap[e] = sgn[c] * S[i * ld + c];
-  }
-}
-
-static bool qr_small_fits(int m, int n) {
-  return m >= n && n >= 1 && n <= 256 && (int64_t)m * (n + 1) <= kQrSmallBig;
-}
-
-static int qr_small_b(double* A, int m, int n, int trans, double* R, int batch, hipStream_t s) {
-  TNX_CHECK_ARG(qr_small_fits(m, n), "qr_batched: %d x %d exceeds the LDS-resident limit", m, n);
-  TNX_CHECK_ARG(batch >= 1 && batch <= 2147483647, "qr_batched: bad batch %d", batch);
-  if ((int64_t)m * (n + 1) <= kQrSmallLittle)
-    hipLaunchKernelGGL(qr_small_kernel<kQrSmallLittle>, dim3(batch), dim3(256), 0, s, A, m, n,
-                       trans, R);
-  else
-    hipLaunchKernelGGL(qr_small_kernel<kQrSmallBig>, dim3(batch), dim3(256), 0, s, A, m, n, trans,
-                       R);
-  TNX_LAUNCH_CHECK();
-  return TNX_OK;
 }
 
 size_t gauge_b_ws_bytes(int chil, int d, int chir, int batch) {
