@@ -1,5 +1,6 @@
-"""The QR of matrices that fit in LDS (Cholesky QR with regularised pivots,
-Householder where it does not converge) and its transposed and batched forms.
+"""Cholesky QR with regularised pivots: matrices that fit in LDS (one
+workgroup), its transposed and batched forms, and larger matrices in wide
+panels; Householder where squares leave the range of the numbers.
 
 Tolerances: Q is formed by one triangular solve from columns orthonormal to
 0.1, so |Q^T Q - I| carries the rounding of m-term and n-term sums, eps (m +
@@ -13,10 +14,12 @@ pytestmark = pytest.mark.gpu
 
 EPS = np.finfo(np.float64).eps
 
-# edges of the 16-wide tiles, of the two LDS sizes and of the largest shapes;
-# the last two are past the limit
+# edges of the 16-wide tiles, of the two LDS sizes and of the largest shapes
 SHAPES = [(1, 1), (2, 1), (16, 16), (17, 16), (33, 17), (64, 32), (65, 33), (96, 48), (48, 48), (120, 60), (128, 64),
-          (144, 72), (80, 80), (1000, 16), (300, 48), (160, 80), (128, 128)]
+          (144, 72), (80, 80), (1000, 16), (300, 48)]
+# past the LDS limit: one panel, edges of a second and a third, long and square
+WIDE = [(160, 80), (128, 128), (129, 129), (500, 100), (257, 131), (259, 259), (520, 257), (600, 300), (401, 399),
+        (5000, 17), (8192, 33), (1200, 640)]
 
 
 def matrix(kind, m, n):
@@ -33,6 +36,11 @@ def matrix(kind, m, n):
         a[:, -1] = a[:, 0]
     elif kind == "zero":
         a[:, n // 3] = 0.0
+        a[:, n // 2:n // 2 + 3] = 0.0
+    elif kind == "null":
+        a[:] = 0.0
+    elif kind in ("huge", "tiny"):  # squares past 1e290 and below 1e-290
+        a *= 1e147 if kind == "huge" else 1e-147
     elif kind == "scaled":  # columns over 200 decades
         a *= 10.0 ** rng.uniform(-100, 100, n)
     return a
@@ -57,10 +65,10 @@ def workspace(nbytes):
     return buf, buf.data_ptr(), nbytes
 
 
-@pytest.mark.parametrize("kind", ["random", "graded", "rank", "equal", "zero", "scaled"])
-@pytest.mark.parametrize("m, n", SHAPES)
-def test_qr_in_lds(gpu, m, n, kind):
-    print(f"qr in LDS {kind} {m}x{n}", flush=True)
+@pytest.mark.parametrize("kind", ["random", "graded", "rank", "equal", "zero", "null", "scaled", "huge", "tiny"])
+@pytest.mark.parametrize("m, n", SHAPES + WIDE)
+def test_qr(gpu, m, n, kind):
+    print(f"qr {kind} {m}x{n}", flush=True)
     L = lib().lib()
     a = matrix(kind, m, n)
     ad, r = torch.from_numpy(a.copy()).cuda(), torch.full((n, n), 7.0, dtype=torch.float64, device="cuda")
@@ -79,10 +87,10 @@ def test_qr_in_lds(gpu, m, n, kind):
 @pytest.mark.parametrize("chi", [7, 24, 60])
 def test_gauge_left_in_lds(gpu, chi):
     """The transposed form, and a batch in which one matrix takes the
-    Householder steps: each the same as its matrix alone."""
+    Householder steps (huge): each the same as its matrix alone."""
     L = lib().lib()
     st = torch.cuda.current_stream().cuda_stream
-    kinds = ["random", "zero", "rank", "graded", "random"]
+    kinds = ["random", "zero", "rank", "graded", "huge", "random"]
     a = np.stack([matrix(k, 2 * chi, chi).T.reshape(chi, 2, chi) * (1 + i) for i, k in enumerate(kinds)])
     prev = np.random.default_rng(chi).standard_normal((len(kinds), 5, chi))
     ad, pd = torch.from_numpy(a.copy()).cuda(), torch.from_numpy(prev).cuda()

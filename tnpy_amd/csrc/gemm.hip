@@ -215,6 +215,7 @@ static GemmArgs args_of(const GemmDesc& d) {
   g.nb2 = d.nb2 > 0 ? d.nb2 : 1;
   g.sA2 = d.sA2; g.sB2 = d.sB2; g.sC2 = d.sC2;
   g.bidx = d.bidx;
+  g.gate = d.gate;
   g.kc = d.K;
   g.partial = nullptr;
   return g;

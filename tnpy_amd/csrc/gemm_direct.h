@@ -228,6 +228,7 @@ struct GemmOperand {
 template <int PREC, int TM, int TN, int WM, int WN, int WK, int PD, int OCC, bool A_K, bool B_N,
           typename TA, typename TB>
 __global__ __launch_bounds__(64 * WM * WN * WK, OCC) void gemm_direct_kernel(GemmArgs g) {
+  if (g.gate && *g.gate == 0) return;
   using acc_t = typename PT<PREC>::acc_t;
   using CT = typename PT<PREC>::lds_t;
   using OA = GemmOperand<TM, A_K, TA>;

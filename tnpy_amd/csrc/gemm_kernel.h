@@ -63,6 +63,7 @@ struct GemmArgs {
   int nb2;          // second batch level (1 = none)
   int64_t sA2, sB2, sC2;
   const int* bidx;  // launched -> logical batch index, or null
+  const int* gate;  // nothing is done when this device flag is 0; or null
 };
 
 // The output tile of this workgroup.
@@ -115,6 +116,7 @@ __device__ __forceinline__ T vec_elem(const u32x4& v, int j) {
 template <int PREC, int BM, int BN, bool A_K, bool B_N, int WGM, int WGN, int BK, typename TA,
           typename TB>
 __global__ __launch_bounds__(64 * WGM * WGN) void gemm_kernel(GemmArgs g) {
+  if (g.gate && *g.gate == 0) return;
   using lds_t = typename PT<PREC>::lds_t;
   using acc_t = typename PT<PREC>::acc_t;
   constexpr bool TYPED = !std::is_void<TA>::value;

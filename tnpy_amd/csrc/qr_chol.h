@@ -9,8 +9,9 @@
 // keeps its components along the earlier ones, scaled up, and the next pass,
 // whose Gram matrix is formed from those scaled columns, resolves it. So
 // graded and numerically rank-deficient matrices need three or four passes
-// instead of two and no other algorithm; only columns that vanish exactly do
-// not converge. P - Q R stays at rounding level in every pass because P is
+// instead of two and no other algorithm. A column that vanishes exactly has a
+// zero row in R and any direction will do for Q: it is filled with
+// pseudo-random numbers after the first pass. P - Q R stays at rounding level in every pass because P is
 // solved against L, not multiplied by its inverse: 16-wide blocks by forward
 // substitution, the inverse only of the diagonal blocks and corrected once by
 // the residual where a block may be ill conditioned.
@@ -35,6 +36,16 @@ constexpr int kQcPasses = 6;
 
 __device__ __forceinline__ qc_f64x4 qc_mfma(double a, double b, qc_f64x4 c) {
   return __builtin_amdgcn_mfma_f64_16x16x4f64(a, b, c, 0, 0, 0);
+}
+
+// Entry (i, c) of the filling of a zero column: even in (-1, 1), from the
+// position alone (splitmix64), so the factorisation is reproducible.
+__device__ __forceinline__ double qc_fill(unsigned i, unsigned c) {
+  unsigned long long z = ((unsigned long long)c << 32 | i) + 0x9e3779b97f4a7c15ull;
+  z = (z ^ (z >> 30)) * 0xbf58476d1ce4e5b9ull;
+  z = (z ^ (z >> 27)) * 0x94d049bb133111ebull;
+  z ^= z >> 31;
+  return (double)(long long)z * 0x1p-63;
 }
 
 // Lane i's value as a wave-uniform scalar; i must be wave-uniform.
@@ -89,8 +100,8 @@ __device__ __forceinline__ void qc_chol16(double (&a)[16], double d0, double tau
 // waves factor the diagonal block of a step (16 columns, no barrier between
 // them), each with up to 32 of the rows below; NT / 2 >= 16 nb.
 // Returns ill (above) for the whole workgroup.
-template <int NT, int nb, int ld>
-__device__ __forceinline__ bool qc_cholesky(double* G, const double* d0, double tau, double* X, int* flag) {
+template <int NT, int ld>
+__device__ __forceinline__ bool qc_cholesky(double* G, int nb, const double* d0, double tau, double* X, int* flag) {
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, lr = lane & 15, lk = lane >> 4;
   constexpr int NW = NT / 64;
   bool ill = false;
@@ -148,10 +159,11 @@ __device__ __forceinline__ bool qc_cholesky(double* G, const double* d0, double 
 // on entry). L (row stride ld) and the diagonal inverses X in LDS or global
 // memory; refine corrects every diagonal solve by its residual.
 template <int NB, int ld>
-__device__ __forceinline__ void qc_trsm(qc_f64x4 (&Z)[NB], const double* L, const double* X, bool refine) {
+__device__ __forceinline__ void qc_trsm(qc_f64x4 (&Z)[NB], int nb, const double* L, const double* X, bool refine) {
   const int lane = threadIdx.x & 63, lr = lane & 15, lk = lane >> 4;
 #pragma unroll
   for (int j = 0; j < NB; ++j) {
+    if (j >= nb) break;
     const double* Lj = L + (16 * j + lr) * ld + lk;
     qc_f64x4 acc = Z[j];
 #pragma unroll

@@ -88,6 +88,9 @@ struct GemmDesc {
   // Optional index list: launched batch i computes logical batch bidx[i]
   // (a subset of a larger stack); null means launched == logical.
   const int* bidx = nullptr;
+  // Optional device flag: the workgroups return at once when it is 0 (a
+  // step that the device decides to leave out).
+  const int* gate = nullptr;
 };
 
 int gemm(const GemmDesc& g, hipStream_t stream);
