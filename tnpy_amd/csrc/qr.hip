@@ -722,9 +722,11 @@ __global__ __launch_bounds__(512) void wp_factor_kernel(WpBuf b, int j0, int w, 
   __shared__ double d0[kWpW];
   __shared__ int sh[3];  // far from I, not close to I, out of range
   __shared__ int flag;
+  __shared__ unsigned zero[4];
   if (p >= 2 && b.flags[p] == 0) return;
   const int tid = threadIdx.x;
   if (tid < 3) sh[tid] = 0;
+  if (tid < 4) zero[tid] = 0;
   __syncthreads();
   bool far = false, wide = false, bad = false;
 #pragma unroll
@@ -733,31 +735,33 @@ __global__ __launch_bounds__(512) void wp_factor_kernel(WpBuf b, int j0, int w, 
 #pragma unroll
     for (int u = 0; u < 16; ++u) {
       const int e = tid + 512 * (16 * h + u), i = e >> 7, c = e & 127;
-      v[u] = i < w && c <= i ? b.S[(size_t)(j0 + i) * kWpW + c] : (i == c ? 1.0 : 0.0);
+      const double x = b.S[(size_t)(j0 + min(i, w - 1)) * kWpW + c];
+      v[u] = i < w && c <= i ? x : (i == c ? 1.0 : 0.0);
     }
 #pragma unroll
     for (int u = 0; u < 16; ++u) {
       const int e = tid + 512 * (16 * h + u), i = e >> 7, c = e & 127;
-      double x = v[u];
-      if (i == c) {
-        if (p == 0 && x == 0.0) {
-          atomicOr(&b.flags[kWpZero + (i >> 5)], 1 << (i & 31));
-          x = 1.0;
-        }
-        d0[i] = x;
-        bad = bad || !(x > 1e-290 && x < 1e290);
-      }
-      const double off = c <= i ? fabs(x - (i == c ? 1.0 : 0.0)) : 0.0;
+      const double off = fabs(v[u] - (i == c ? 1.0 : 0.0));
       far = far || !(off <= 0.1);
       wide = wide || !(off <= 1e-9);
-      G[i * kWpLd + c] = x;
+      G[i * kWpLd + c] = v[u];
     }
+  }
+  __syncthreads();
+  if (tid < kWpW) {
+    double x = G[tid * kWpLd + tid];
+    if (p == 0 && x == 0.0) {
+      atomicOr(&zero[tid >> 5], 1u << (tid & 31));
+      x = G[tid * kWpLd + tid] = 1.0;
+    }
+    d0[tid] = x;
+    bad = !(x > 1e-290 && x < 1e290);
   }
   if (far) sh[0] = 1;
   if (wide) sh[1] = 1;
   if (bad) sh[2] = 1;
-  __threadfence();
   __syncthreads();
+  if (p == 0 && tid < 4) b.flags[kWpZero + tid] = (int)zero[tid];
   if (tid == 0) {
     if (sh[2]) b.flags[kWpPasses] = 1;
     if (p >= 1 && sh[0]) b.flags[p + 1] = 1;
@@ -783,14 +787,10 @@ __global__ __launch_bounds__(512) void wp_factor_kernel(WpBuf b, int j0, int w, 
     b.L[e] = c <= i ? G[i * kWpLd + c] : 0.0;
   }
   if (p == 0) {
-    unsigned z[4];
-#pragma unroll
-    for (int q = 0; q < 4; ++q) z[q] = (unsigned)atomicAdd(&b.flags[kWpZero + q], 0);
 #pragma unroll 8
     for (int e = tid; e < kWpW * kWpW; e += 512) {
       const int i = e >> 7, c = e & 127;
-      const unsigned zi = i < 64 ? (i < 32 ? z[0] : z[1]) : (i < 96 ? z[2] : z[3]);
-      b.Rp[0][e] = c >= i && !(zi >> (i & 31) & 1) ? G[c * kWpLd + i] : 0.0;
+      b.Rp[0][e] = c >= i && !(zero[i >> 5] >> (i & 31) & 1) ? G[c * kWpLd + i] : 0.0;
     }
   }
   for (int e = tid; e < kWpW * kQcXLd; e += 512) b.X[e] = X[e];
@@ -809,12 +809,45 @@ __global__ __launch_bounds__(256) void wp_rows_kernel(double* __restrict__ A, in
   const int nb = (w + 15) / 16, nc = (j0 + 63) / 64, blk = blockIdx.x;
   const bool rows = blk < nrow, crow = !rows && blk < nrow + nc;
   const double* Ro = b.Rp[(p - 1) & 1];
+  const int r0 = 64 * (rows ? blk : blk - nrow) + 16 * wave, row = r0 + lr;
+  const int cb = 4 * (blk - nrow - nc) + wave;  // block column of R_p
+  const bool in = row < (rows ? m : j0);        // j0 is a whole number of tiles
+  double* Ap = (rows ? A : R) + (int64_t)(in ? row : 0) * n + j0 + lk;
+  qc_f64x4 Z[kWpNB], Y[kWpNB];
+  int ill = 0, z[4];
   {
     // the 36 tiles of L's lower triangle, or R_p's upper one for the rows of
-    // C, with all loads in flight before the first LDS store
+    // C, the diagonal inverses and the rows of P: all loads in flight before
+    // the first LDS store
+    ill = b.flags[kWpIll];
+#pragma unroll
+    for (int q = 0; q < 4; ++q) z[q] = b.flags[kWpZero + q];
     const double* src = crow ? Ro : b.L;
-    double t[36];
-    constexpr int kT = kWpNB * (kWpNB + 1) / 2;
+    constexpr int kX = (kWpW * kQcXLd + 255) / 256, kT = kWpNB * (kWpNB + 1) / 2;
+    double t[kT], x[kX];
+    if (rows) {
+#pragma unroll
+      for (int u = 0; u < kX; ++u) x[u] = b.X[min(tid + 256 * u, kWpW * kQcXLd - 1)];
+    }
+    if (rows || crow) {
+      // the rows of P, or of C with those of R_<p
+      const double* Cp = b.S + (size_t)(in ? row : 0) * kWpW + lk;
+#pragma unroll
+      for (int j = 0; j < kWpNB; ++j)
+#pragma unroll
+        for (int v = 0; v < 4; ++v) {
+          const int c = 16 * j + 4 * v;
+          const bool on = in && c + lk < w;
+          const double a = Ap[min(c, w - 1 - lk)], e = crow ? Cp[c] : 0.0;
+          Z[j][v] = on ? (crow ? e : a) : 0.0;
+          Y[j][v] = on ? a : 0.0;
+        }
+    } else {
+#pragma unroll
+      for (int k = 0; k < kWpNB; ++k)
+#pragma unroll
+        for (int v = 0; v < 4; ++v) Z[k][v] = k <= cb ? Ro[(16 * k + lk + 4 * v) * kWpW + 16 * (cb & 7) + lr] : 0.0;
+    }
 #pragma unroll
     for (int bi = 0, q = 0; bi < kWpNB; ++bi)
 #pragma unroll
@@ -822,7 +855,6 @@ __global__ __launch_bounds__(256) void wp_rows_kernel(double* __restrict__ A, in
         const int r = crow ? bj : bi, c = crow ? bi : bj;
         t[q] = bi < nb ? src[(16 * r + (tid >> 4)) * kWpW + 16 * c + (tid & 15)] : 0.0;
       }
-    static_assert(kT == 36, "tiles of the triangle");
 #pragma unroll
     for (int bi = 0, q = 0; bi < kWpNB; ++bi)
 #pragma unroll
@@ -830,23 +862,17 @@ __global__ __launch_bounds__(256) void wp_rows_kernel(double* __restrict__ A, in
         const int r = crow ? bj : bi, c = crow ? bi : bj;
         T[(16 * r + (tid >> 4)) * kWpLd + 16 * c + (tid & 15)] = t[q];
       }
-    if (rows)
-      for (int e = tid; e < kWpW * kQcXLd; e += 256) X[e] = b.X[e];
+    if (rows) {
+#pragma unroll
+      for (int u = 0; u < kX; ++u)
+        if (tid + 256 * u < kWpW * kQcXLd) X[tid + 256 * u] = x[u];
+    }
   }
   __syncthreads();
   if (rows) {
-    const int row = 64 * blk + 16 * wave + lr;
-    if (64 * blk + 16 * wave >= m) return;
-    double* Ap = A + (int64_t)row * n + j0 + lk;
-    const bool in = row < m;
-    qc_f64x4 Z[kWpNB];
-#pragma unroll
-    for (int j = 0; j < kWpNB; ++j)
-#pragma unroll
-      for (int v = 0; v < 4; ++v) Z[j][v] = in && 16 * j + 4 * v + lk < w ? Ap[16 * j + 4 * v] : 0.0;
-    qc_trsm<kWpNB, kWpLd>(Z, nb, T, X, b.flags[kWpIll] != 0);
+    if (r0 >= m) return;
+    qc_trsm<kWpNB, kWpLd>(Z, nb, T, X, ill != 0);
     if (p == 0) {
-      const int* z = b.flags + kWpZero;
       if (z[0] | z[1] | z[2] | z[3]) {
         const double sc = sqrt(3.0 / m);
 #pragma unroll
@@ -854,7 +880,7 @@ __global__ __launch_bounds__(256) void wp_rows_kernel(double* __restrict__ A, in
 #pragma unroll
           for (int v = 0; v < 4; ++v) {
             const int c = 16 * j + 4 * v + lk;
-            if ((unsigned)z[c >> 5] >> (c & 31) & 1) Z[j][v] = sc * qc_fill(row, j0 + c);
+            if ((unsigned)z[j >> 1] >> (c & 31) & 1) Z[j][v] = sc * qc_fill(row, j0 + c);
           }
       }
     }
@@ -866,54 +892,38 @@ __global__ __launch_bounds__(256) void wp_rows_kernel(double* __restrict__ A, in
     return;
   }
   if (crow) {
-    const int r0 = 64 * (blk - nrow) + 16 * wave;
-    if (r0 >= j0) return;  // j0 is a whole number of tiles
-    const double* Cp = b.S + (size_t)(r0 + lr) * kWpW + lk;
-    double* Rr = R + (int64_t)(r0 + lr) * n + j0 + lk;
-    qc_f64x4 Z[kWpNB];
+    if (r0 >= j0) return;
     bool far = false;
 #pragma unroll
     for (int j = 0; j < kWpNB; ++j)
 #pragma unroll
-      for (int v = 0; v < 4; ++v) {
-        Z[j][v] = 16 * j + 4 * v + lk < w ? Cp[16 * j + 4 * v] : 0.0;
-        far = far || !(fabs(Z[j][v]) <= kWpFar);
-      }
+      for (int v = 0; v < 4; ++v) far = far || !(fabs(Z[j][v]) <= kWpFar);
     if (far) b.flags[p + 1] = 1;
 #pragma unroll
     for (int j = 0; j < kWpNB; ++j) {
       if (j >= nb) break;
-      qc_f64x4 acc;
-#pragma unroll
-      for (int v = 0; v < 4; ++v) acc[v] = 16 * j + 4 * v + lk < w ? Rr[16 * j + 4 * v] : 0.0;
 #pragma unroll
       for (int k = 0; k <= j; ++k)
 #pragma unroll
         for (int kk = 0; kk < 4; ++kk)
-          acc = qc_mfma(T[(16 * k + 4 * kk + lk) * kWpLd + 16 * j + lr], Z[k][kk], acc);
+          Y[j] = qc_mfma(T[(16 * k + 4 * kk + lk) * kWpLd + 16 * j + lr], Z[k][kk], Y[j]);
 #pragma unroll
       for (int v = 0; v < 4; ++v)
-        if (16 * j + 4 * v + lk < w) Rr[16 * j + 4 * v] = acc[v];
+        if (16 * j + 4 * v + lk < w) Ap[16 * j + 4 * v] = Y[j][v];
       __builtin_amdgcn_sched_barrier(0);
     }
     return;
   }
-  const int cb = 4 * (blk - nrow - nc) + wave;
   if (cb >= nb) return;
-  qc_f64x4 Rb[kWpNB];
-#pragma unroll
-  for (int k = 0; k < kWpNB; ++k)
-#pragma unroll
-    for (int v = 0; v < 4; ++v) Rb[k][v] = k <= cb ? Ro[(16 * k + lk + 4 * v) * kWpW + 16 * cb + lr] : 0.0;
-  qc_update_r<kWpNB, kWpLd>(Rb, cb, T);
+  qc_update_r<kWpNB, kWpLd>(Z, cb, T);
   double* Rn = b.Rp[p & 1];
 #pragma unroll
   for (int k = 0; k < kWpNB; ++k)
 #pragma unroll
     for (int v = 0; v < 4; ++v) {
       const int i = 16 * k + lk + 4 * v, c = 16 * cb + lr;
-      Rn[i * kWpW + c] = Rb[k][v];
-      if (i < w && c < w) R[(int64_t)(j0 + i) * n + j0 + c] = Rb[k][v];
+      Rn[i * kWpW + c] = Z[k][v];
+      if (i < w && c < w) R[(int64_t)(j0 + i) * n + j0 + c] = Z[k][v];
     }
 }
 

@@ -64,33 +64,32 @@ __device__ __forceinline__ double qc_lane(double v, int i) {
 __device__ __forceinline__ void qc_chol16(double (&a)[16], double d0, double tau, bool& ill) {
   const int lane = threadIdx.x & 63;
   const bool inv = lane >= 16 && lane < 32;
-  // the pivot of step j + 1 is ready after one of step j's updates, so its
-  // reciprocal root overlaps the rest of them
-  bool ok;
-  double d, rs;
+  // The pivot of step j + 1 is ready after one of step j's updates, so its
+  // reciprocal root overlaps the rest of them. Selects, no branches: those
+  // would split the register array. (Bound by instruction issue, 270 cycles a
+  // column. The multipliers through LDS instead of lane reads took as long,
+  // and an LDL^T form with one root at the end 330.)
+  double d, rs, mul, low = 1.0;
   auto pivot = [&](int j) {
-    const double g0 = qc_lane(d0, j);
-    const double thr = tau * g0;
-    d = qc_lane(a[j], j);
-    ok = d > thr;
-    ill = ill || !(d > 1e-2 * g0);
-    d = ok ? d : thr;
+    const double g0 = qc_lane(d0, j), x = qc_lane(a[j], j), thr = tau * g0;
+    d = fmax(x, thr);
     rs = rsqrt_nr(d);
+    mul = inv || x > thr ? rs : 0.0;
+    low = fmin(low, fma(-1e-2, g0, x));
   };
   pivot(0);
 #pragma unroll
   for (int j = 0; j < 16; ++j) {
-    const double sc = a[j] * rs;
-    const bool go = ok;
-    a[j] = lane == j ? d * rs : (go || inv ? sc : 0.0);
+    a[j] = lane == j ? d * rs : a[j] * mul;
     if (j + 1 < 16) {
-      a[j + 1] = fma(-a[j], go ? qc_lane(sc, j + 1) : 0.0, a[j + 1]);
+      a[j + 1] = fma(-a[j], qc_lane(a[j], j + 1), a[j + 1]);
       pivot(j + 1);
     }
 #pragma unroll
-    for (int c = j + 2; c < 16; ++c) a[c] = fma(-a[j], go ? qc_lane(sc, c) : 0.0, a[c]);
+    for (int c = j + 2; c < 16; ++c) a[c] = fma(-a[j], qc_lane(a[j], c), a[c]);
     __builtin_amdgcn_sched_barrier(0);
   }
+  ill = ill || !(low > 0.0);
 }
 
 // Cholesky factor of the 16 nb x 16 nb matrix in LDS (lower triangle of G, row
@@ -106,48 +105,56 @@ __device__ __forceinline__ bool qc_cholesky(double* G, int nb, const double* d0,
   constexpr int NW = NT / 64;
   bool ill = false;
   if (tid == 0) *flag = 0;
+  // tile (i, j) minus the product of its rows in block column kb
+  auto update = [&](int i, int j, int kb) {
+    const double* Gi = G + (16 * i + lr) * ld + 16 * kb + lk;
+    const double* Gj = G + (16 * j + lr) * ld + 16 * kb + lk;
+    double* C = G + (16 * i + lk) * ld + 16 * j + lr;
+    qc_f64x4 g;
+#pragma unroll
+    for (int v = 0; v < 4; ++v) g[v] = C[4 * v * ld];
+#pragma unroll
+    for (int kk = 0; kk < 4; ++kk) g = qc_mfma(-Gi[4 * kk], Gj[4 * kk], g);
+#pragma unroll
+    for (int v = 0; v < 4; ++v) C[4 * v * ld] = g[v];
+  };
   for (int kb = 0; kb < nb; ++kb) {
     const int base = 16 * kb, below = base + 16 + 32 * wave;
     const int row = lane < 16 ? base + lane : below + lane - 32;
     const bool on = lane < 16 || (lane >= 32 && row < 16 * nb);
-    const bool busy = wave == 0 || below < 16 * nb;
+    const int nf = max(1, (16 * (nb - kb - 1) + 31) / 32);  // waves with rows
     double a[16];
-    if (busy) {
+    if (wave < nf) {
+      const double* src = G + (on ? row : base) * ld + base;
 #pragma unroll
-      for (int c = 0; c < 16; ++c)
-        a[c] = on ? G[row * ld + base + c] : (lane - 16 == c ? 1.0 : 0.0);
-    }
-    __syncthreads();
-    if (busy) {
+      for (int c = 0; c < 16; ++c) {
+        const double x = src[c];
+        a[c] = on ? x : (lane - 16 == c ? 1.0 : 0.0);
+      }
       qc_chol16(a, lane < 16 ? d0[base + lane] : 0.0, tau, ill);
       if (lane >= 32 && on) {
 #pragma unroll
         for (int c = 0; c < 16; ++c) G[row * ld + base + c] = a[c];
       }
-      if (wave == 0 && lane < 16) {
-#pragma unroll
-        for (int c = 0; c < 16; ++c) G[row * ld + base + c] = c <= lane ? a[c] : 0.0;
-      }
-      if (wave == 0 && lane >= 16 && lane < 32) {
-#pragma unroll
-        for (int r = 0; r < 16; ++r) X[(base + r) * kQcXLd + lane - 16] = a[r];
+    } else if (kb > 0) {
+      // the other waves meanwhile finish the update by the block column before
+      const int left = nb - kb - 1, tiles = left * (left + 1) / 2;
+      for (int t = wave - nf; t < tiles; t += NW - nf) {
+        int i = 0, j = t;
+        while (j > i) { j -= i + 1; ++i; }
+        update(kb + 1 + i, kb + 1 + j, kb - 1);
       }
     }
     __syncthreads();
-    const int left = nb - kb - 1, tiles = left * (left + 1) / 2;
-    for (int t = wave; t < tiles; t += NW) {
-      int i = 0, rem = t;
-      while (rem > i) { rem -= i + 1; ++i; }
-      const int i0 = base + 16 + 16 * i, j0 = base + 16 + 16 * rem;
-      qc_f64x4 g;
+    // every wave has read the diagonal block, and the updates do not
+    if (wave == 0 && lane < 32) {
+      double* dst = lane < 16 ? G + row * ld + base : X + base * kQcXLd + lane - 16;
+      const int step = lane < 16 ? 1 : kQcXLd;
 #pragma unroll
-      for (int v = 0; v < 4; ++v) g[v] = G[(i0 + lk + 4 * v) * ld + j0 + lr];
-#pragma unroll
-      for (int kk = 0; kk < 4; ++kk)
-        g = qc_mfma(-G[(i0 + lr) * ld + base + 4 * kk + lk], G[(j0 + lr) * ld + base + 4 * kk + lk], g);
-#pragma unroll
-      for (int v = 0; v < 4; ++v) G[(i0 + lk + 4 * v) * ld + j0 + lr] = g[v];
+      for (int c = 0; c < 16; ++c) dst[c * step] = lane >= 16 || c <= lane ? a[c] : 0.0;
     }
+    // what the next step factors: block column kb + 1
+    for (int i = kb + 1 + (NW - 1 - wave); i < nb; i += NW) update(i, kb + 1, kb);
     __syncthreads();
   }
   if (ill && wave == 0 && lane == 0) *flag = 1;
