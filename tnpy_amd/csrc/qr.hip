@@ -579,7 +579,7 @@ __global__ __launch_bounds__(NT) void qr_chol_kernel(double* __restrict__ A, int
         for (int k = 0; k < NB; ++k)
 #pragma unroll
           for (int v = 0; v < 4; ++v) {
-            const int i = 16 * k + lk + 4 * v;
+            const int i = 16 * k + 4 * lk + v;
             const bool on = k <= wave && !(zero[i >> 5] >> (i & 31) & 1);
             Rb[k][v] = on ? G[(16 * wave + lr) * ld + i] : 0.0;
           }
@@ -588,17 +588,17 @@ __global__ __launch_bounds__(NT) void qr_chol_kernel(double* __restrict__ A, int
       }
     }
     for (int t = wave; t < mt; t += NW) {
-      double* St = S + (16 * t + lr) * ld + lk;
+      double* St = S + (16 * t + lr) * ld + 4 * lk;
       qc_f64x4 Z[NB];
 #pragma unroll
       for (int j = 0; j < NB; ++j)
 #pragma unroll
-        for (int v = 0; v < 4; ++v) Z[j][v] = St[16 * j + 4 * v];
+        for (int v = 0; v < 4; ++v) Z[j][v] = St[16 * j + v];
       qc_trsm<NB, ld>(Z, NB, G, X, ill);
 #pragma unroll
       for (int j = 0; j < NB; ++j)
 #pragma unroll
-        for (int v = 0; v < 4; ++v) St[16 * j + 4 * v] = Z[j][v];
+        for (int v = 0; v < 4; ++v) St[16 * j + v] = Z[j][v];
     }
     __syncthreads();
     if (p == 0 && (zero[0] | zero[1] | zero[2])) {
@@ -618,7 +618,7 @@ __global__ __launch_bounds__(NT) void qr_chol_kernel(double* __restrict__ A, int
     for (int k = 0; k < NB; ++k)
 #pragma unroll
       for (int v = 0; v < 4; ++v) {
-        const int i = 16 * k + lk + 4 * v;
+        const int i = 16 * k + 4 * lk + v;
         if (i < n && c < n) Rp[i * n + c] = Rb[k][v];
       }
   }
@@ -688,20 +688,23 @@ static int qr_small_b(double* A, int m, int n, int trans, double* R, int batch, 
 //   pass 0:   G = P^T P, P <- P L^-T;
 //   pass 1:   [C; G] = [Q_<  P]^T P, P <- (P - Q_< C) L^-T,
 //             R_<p += C R_p, R_p <- L^T R_p;
-//   pass 2, 3: the same again, left out on the device once a pass has started
-//             from |G - I| <= 0.1 and |C| <= kWpFar (then the C^T C that G
-//             leaves out is below rounding);
+//   pass 2, 3: the same again, needed while the pass before has started from
+//             |G - I| > 0.1 or |C| > kWpFar (below it the C^T C that G leaves
+//             out is at rounding level: its n terms are squares of entries
+//             that are well below the largest);
 //   then R_p,> = P^T A_> and A_> -= P R_p,> for the columns behind.
 // Q replaces A in place and needs no backward formation, so a panel costs one
 // workgroup's 128-wide factorisation (wp_factor) and GEMMs, where 32-wide
 // Householder panels took four of everything and rebuilt their reflectors.
 // Well-conditioned panels take two passes, graded and rank-deficient ones
-// three or four (zero columns included, see qc_fill); what does not converge
-// (numbers out of the Gram matrix's range) sets the panel's last flag and the
-// host factors the saved copy by Householder panels.
+// three or four (zero columns included, see qc_fill). The host queues two, and
+// from the saved copy all four where a panel has asked for them; a panel then
+// leaves out on the device what it does not need, for 4.5 us a launch (280 us
+// at n = 1024, why they are not queued at once). What does not converge in four
+// (numbers out of the Gram matrix's range) is factored by Householder panels.
 constexpr int kWpW = 128, kWpNB = kWpW / 16, kWpLd = kWpW + 1;
 constexpr int kWpPasses = 4;
-constexpr double kWpFar = 3e-10;
+constexpr double kWpFar = 2e-9;
 // flags of a panel: [p] pass p is needed (p = 2, 3), [kWpPasses] it did not
 // converge, [kWpIll] the current factor's ill, [kWpZero ..] zero columns
 constexpr int kWpIll = 6, kWpZero = 8, kWpFlags = 16;
@@ -800,7 +803,7 @@ __global__ __launch_bounds__(512) void wp_factor_kernel(WpBuf b, int j0, int w, 
 // rows of P against L; the next ones, from pass 1 on, take C's rows, R_<p += C
 // R_p, and ask for another pass where C is not small; the last two take R_p <-
 // L^T R_p, one block column per wave.
-__global__ __launch_bounds__(256) void wp_rows_kernel(double* __restrict__ A, int m, int n, int j0, int w,
+__global__ __launch_bounds__(256) void wp_rows_kernel(double* __restrict__ A, int m, int n, int j0, int w, bool pairs,
                                                       double* __restrict__ R, WpBuf b, int p, int nrow) {
   __shared__ double T[kWpW * kWpLd];
   __shared__ double X[kWpW * kQcXLd];
@@ -812,7 +815,7 @@ __global__ __launch_bounds__(256) void wp_rows_kernel(double* __restrict__ A, in
   const int r0 = 64 * (rows ? blk : blk - nrow) + 16 * wave, row = r0 + lr;
   const int cb = 4 * (blk - nrow - nc) + wave;  // block column of R_p
   const bool in = row < (rows ? m : j0);        // j0 is a whole number of tiles
-  double* Ap = (rows ? A : R) + (int64_t)(in ? row : 0) * n + j0 + lk;
+  double* Ap = (rows ? A : R) + (int64_t)(in ? row : 0) * n + j0 + 4 * lk;
   qc_f64x4 Z[kWpNB], Y[kWpNB];
   int ill = 0, z[4];
   {
@@ -831,22 +834,34 @@ __global__ __launch_bounds__(256) void wp_rows_kernel(double* __restrict__ A, in
     }
     if (rows || crow) {
       // the rows of P, or of C with those of R_<p
-      const double* Cp = b.S + (size_t)(in ? row : 0) * kWpW + lk;
+      const double* Cp = b.S + (size_t)(in ? row : 0) * kWpW + 4 * lk;
 #pragma unroll
-      for (int j = 0; j < kWpNB; ++j)
+      for (int j = 0; j < kWpNB; ++j) {
+        qc_f64x4 a, e = {0.0, 0.0, 0.0, 0.0};
+        if (pairs) {  // rows of whole blocks on even places: two loads each
+          const double* Aj = Ap + min(16 * j, w - 16);
+          const qc_f64x2 a0 = *reinterpret_cast<const qc_f64x2*>(Aj), a1 = *reinterpret_cast<const qc_f64x2*>(Aj + 2);
+          a = qc_f64x4{a0[0], a0[1], a1[0], a1[1]};
+        } else {
+#pragma unroll
+          for (int v = 0; v < 4; ++v) a[v] = Ap[min(16 * j + v, w - 1 - 4 * lk)];
+        }
+        if (crow) {
+#pragma unroll
+          for (int v = 0; v < 4; ++v) e[v] = Cp[16 * j + v];
+        }
 #pragma unroll
         for (int v = 0; v < 4; ++v) {
-          const int c = 16 * j + 4 * v;
-          const bool on = in && c + lk < w;
-          const double a = Ap[min(c, w - 1 - lk)], e = crow ? Cp[c] : 0.0;
-          Z[j][v] = on ? (crow ? e : a) : 0.0;
-          Y[j][v] = on ? a : 0.0;
+          const bool on = in && 16 * j + 4 * lk + v < w;
+          Z[j][v] = on ? (crow ? e[v] : a[v]) : 0.0;
+          Y[j][v] = on ? a[v] : 0.0;
         }
+      }
     } else {
 #pragma unroll
       for (int k = 0; k < kWpNB; ++k)
 #pragma unroll
-        for (int v = 0; v < 4; ++v) Z[k][v] = k <= cb ? Ro[(16 * k + lk + 4 * v) * kWpW + 16 * (cb & 7) + lr] : 0.0;
+        for (int v = 0; v < 4; ++v) Z[k][v] = k <= cb ? Ro[(16 * k + 4 * lk + v) * kWpW + 16 * (cb & 7) + lr] : 0.0;
     }
 #pragma unroll
     for (int bi = 0, q = 0; bi < kWpNB; ++bi)
@@ -869,6 +884,21 @@ __global__ __launch_bounds__(256) void wp_rows_kernel(double* __restrict__ A, in
     }
   }
   __syncthreads();
+  auto put = [&](const qc_f64x4(&V)[kWpNB]) {
+#pragma unroll
+    for (int j = 0; j < kWpNB; ++j) {
+      if (pairs) {
+        if (in && 16 * j < w) {
+          *reinterpret_cast<qc_f64x2*>(Ap + 16 * j) = qc_f64x2{V[j][0], V[j][1]};
+          *reinterpret_cast<qc_f64x2*>(Ap + 16 * j + 2) = qc_f64x2{V[j][2], V[j][3]};
+        }
+      } else {
+#pragma unroll
+        for (int v = 0; v < 4; ++v)
+          if (in && 16 * j + 4 * lk + v < w) Ap[16 * j + v] = V[j][v];
+      }
+    }
+  };
   if (rows) {
     if (r0 >= m) return;
     qc_trsm<kWpNB, kWpLd>(Z, nb, T, X, ill != 0);
@@ -879,16 +909,12 @@ __global__ __launch_bounds__(256) void wp_rows_kernel(double* __restrict__ A, in
         for (int j = 0; j < kWpNB; ++j)
 #pragma unroll
           for (int v = 0; v < 4; ++v) {
-            const int c = 16 * j + 4 * v + lk;
+            const int c = 16 * j + 4 * lk + v;
             if ((unsigned)z[j >> 1] >> (c & 31) & 1) Z[j][v] = sc * qc_fill(row, j0 + c);
           }
       }
     }
-#pragma unroll
-    for (int j = 0; j < kWpNB; ++j)
-#pragma unroll
-      for (int v = 0; v < 4; ++v)
-        if (in && 16 * j + 4 * v + lk < w) Ap[16 * j + 4 * v] = Z[j][v];
+    put(Z);
     return;
   }
   if (crow) {
@@ -906,12 +932,10 @@ __global__ __launch_bounds__(256) void wp_rows_kernel(double* __restrict__ A, in
       for (int k = 0; k <= j; ++k)
 #pragma unroll
         for (int kk = 0; kk < 4; ++kk)
-          Y[j] = qc_mfma(T[(16 * k + 4 * kk + lk) * kWpLd + 16 * j + lr], Z[k][kk], Y[j]);
-#pragma unroll
-      for (int v = 0; v < 4; ++v)
-        if (16 * j + 4 * v + lk < w) Ap[16 * j + 4 * v] = Y[j][v];
+          Y[j] = qc_mfma(T[(16 * k + 4 * lk + kk) * kWpLd + 16 * j + qc_at(lr)], Z[k][kk], Y[j]);
       __builtin_amdgcn_sched_barrier(0);
     }
+    put(Y);
     return;
   }
   if (cb >= nb) return;
@@ -921,7 +945,7 @@ __global__ __launch_bounds__(256) void wp_rows_kernel(double* __restrict__ A, in
   for (int k = 0; k < kWpNB; ++k)
 #pragma unroll
     for (int v = 0; v < 4; ++v) {
-      const int i = 16 * k + lk + 4 * v, c = 16 * cb + lr;
+      const int i = 16 * k + 4 * lk + v, c = 16 * cb + lr;
       Rn[i * kWpW + c] = Z[k][v];
       if (i < w && c < w) R[(int64_t)(j0 + i) * n + j0 + c] = Z[k][v];
     }
@@ -944,7 +968,7 @@ static size_t wp_ws_bytes(int n) {
 }
 
 // Queues the factorisation; flags is the device array of every panel's flags.
-static int wp_queue(double* A, int m, int n, double* R, void* ws, int** flags, hipStream_t s) {
+static int wp_queue(double* A, int m, int n, double* R, void* ws, int passes, int** flags, hipStream_t s) {
   char* p = (char*)ws;
   WpBuf b;
   b.S = (double*)p; p += al((size_t)n * kWpW * 8);
@@ -964,8 +988,11 @@ static int wp_queue(double* A, int m, int n, double* R, void* ws, int** flags, h
   t.ta = t.tb = t.tc = DT::F64;
   for (int j0 = 0, pi = 0; j0 < n; j0 += width, ++pi) {
     const int w = std::min(width, n - j0), nt = n - j0 - w;
+    // 16-byte accesses: whole blocks, even row starts in A and R (R and the
+    // other buffers are 256-byte aligned when the caller's A and R are)
+    const bool pairs = w % 16 == 0 && n % 2 == 0 && (((uintptr_t)A | (uintptr_t)R) & 15) == 0;
     b.flags = *flags + pi * kWpFlags;
-    for (int q = 0; q < kWpPasses; ++q) {
+    for (int q = 0; q < passes; ++q) {
       const int top = q == 0 ? j0 : 0;  // the first pass has no use for C
       GemmDesc g = t;
       g.gate = q >= 2 ? b.flags + q : nullptr;
@@ -988,7 +1015,7 @@ static int wp_queue(double* A, int m, int n, double* R, void* ws, int** flags, h
         TNX_TRY(gemm(u, s));
       }
       const int nrow = (m + 63) / 64, more = q > 0 ? (j0 + 63) / 64 + 2 : 0;
-      hipLaunchKernelGGL(wp_rows_kernel, dim3(nrow + more), dim3(256), 0, s, A, m, n, j0, w, R, b, q, nrow);
+      hipLaunchKernelGGL(wp_rows_kernel, dim3(nrow + more), dim3(256), 0, s, A, m, n, j0, w, pairs, R, b, q, nrow);
       TNX_LAUNCH_CHECK();
     }
     if (nt <= 0) continue;
@@ -1018,8 +1045,8 @@ size_t qr_ws_bytes(int m, int n) {
 
 // QR, then what uses Q and R (`after` queues it on the same stream). The wide
 // panels' flags go to a pinned block behind the last panel; the host waits for
-// them with `after` already queued, and queues it again in the rare case that
-// A had to be factored a second time.
+// them with `after` already queued, and queues it again where A had to be
+// factored a second time.
 template <class After>
 static int qr_then(double* A, int m, int n, double* R, void* ws, size_t ws_bytes, hipStream_t s, After after) {
   TNX_CHECK_ARG(A && R, "qr: null pointer");
@@ -1037,37 +1064,45 @@ static int qr_then(double* A, int m, int n, double* R, void* ws, size_t ws_bytes
   char* p = (char*)(((uintptr_t)ws + 255) & ~(uintptr_t)255);
   double* save = (double*)p; p += al((size_t)m * n * 8);
   TNX_TRY(copy_f64(A, save, (int64_t)m * n, s));
-  int* flags = nullptr;
-  TNX_TRY(wp_queue(A, m, n, R, p, &flags, s));
+  // A thread whose last matrix took more than two passes queues all four at
+  // once (the same kind of matrix again, mostly): the results are the same.
+  static thread_local bool more = false;
   const int nf = wp_panels(n) * kWpFlags;
   PinnedLease pin((size_t)(nf + 1) / 2);
   StepEvent fev;
   std::vector<int> plain;
   int* hf = reinterpret_cast<int*>(pin.get());
-  bool queued = false;
-  if (hf && fev.e) {
-    TNX_HIP(hipMemcpyAsync(hf, flags, (size_t)nf * sizeof(int), hipMemcpyDeviceToHost, s));
-    TNX_HIP(hipEventRecord(fev.e, s));
-    const int st = after();
-    // the copy must land before the block goes back to the pool
-    const hipError_t we = hipEventSynchronize(fev.e);
-    TNX_TRY(st);
-    TNX_HIP(we);
-    queued = true;
-  } else {
+  if (!hf || !fev.e) {
     plain.resize(nf);
     hf = plain.data();
+  }
+  auto any = [&](int f) {
+    for (int i = f; i < nf; i += kWpFlags)
+      if (hf[i] != 0) return true;
+    return false;
+  };
+  for (bool four = more;; four = true) {
+    int* flags = nullptr;
+    TNX_TRY(wp_queue(A, m, n, R, p, four ? kWpPasses : 2, &flags, s));
     TNX_HIP(hipMemcpyAsync(hf, flags, (size_t)nf * sizeof(int), hipMemcpyDeviceToHost, s));
-    TNX_HIP(hipStreamSynchronize(s));
-  }
-  bool failed = false;
-  for (int i = kWpPasses; i < nf; i += kWpFlags) failed = failed || hf[i] != 0;
-  if (failed) {
+    if (plain.empty()) {
+      TNX_HIP(hipEventRecord(fev.e, s));
+      const int st = after();
+      // the copy must land before the block goes back to the pool
+      const hipError_t we = hipEventSynchronize(fev.e);
+      TNX_TRY(st);
+      TNX_HIP(we);
+    } else {
+      TNX_HIP(hipStreamSynchronize(s));
+    }
+    more = any(2) || any(kWpPasses);
+    const bool failed = four ? any(kWpPasses) : more;
+    if (!failed) return plain.empty() ? TNX_OK : after();
     TNX_TRY(copy_f64(save, A, (int64_t)m * n, s));
-    TNX_TRY(qr_householder(A, m, n, R, p, s));
-    queued = false;
+    if (four) break;
   }
-  return queued ? TNX_OK : after();
+  TNX_TRY(qr_householder(A, m, n, R, p, s));
+  return after();
 }
 
 int qr(double* A, int m, int n, double* R, void* ws, size_t ws_bytes, hipStream_t s) {
