@@ -785,7 +785,7 @@ __device__ __forceinline__ void tridiag_lowest_wave(TriLds& t, const double* __r
                                     double* __restrict__ s, double* st, int hinted) {
   const int lane = threadIdx.x;
   // the previous call's theta (st[0]), read before this call overwrites it
-  const double hint_in = hinted ? st[0] : 0.0;
+  double hint_in = hinted ? st[0] : 0.0;
   double ar[NC], bl[NC], bn[NC];  // a_k, b_{k-1}, b_k
   double lo = 1e308, hi = 1e308, tnorm = 0.0;
 #pragma unroll
@@ -809,6 +809,24 @@ __device__ __forceinline__ void tridiag_lowest_wave(TriLds& t, const double* __r
     lo = fmin(lo, __shfl_xor(lo, o, 64));
     hi = fmin(hi, __shfl_xor(hi, o, 64));
     tnorm = fmax(tnorm, __shfl_xor(tnorm, o, 64));
+  }
+  // far from 1 the products of rows would leave the range: by a power of two
+  int ex = __builtin_amdgcn_frexp_exp(tnorm);
+  if (ex < -64 || ex > 64) {
+    lo = ldexp(lo, -ex);
+    hi = ldexp(hi, -ex);
+    tnorm = ldexp(tnorm, -ex);
+    hint_in = ldexp(hint_in, -ex);
+#pragma unroll
+    for (int c = 0; c < NC; ++c) {
+      ar[c] = ldexp(ar[c], -ex);
+      bn[c] = ldexp(bn[c], -ex);
+      bl[c] = ldexp(bl[c], -ex);
+      t.row[64 * c + lane] = make_double2(ar[c], bl[c] * bl[c]);
+    }
+    wave_lds_fence();
+  } else {
+    ex = 0;
   }
   const double pivmin = fmax(tnorm, 1e-300) * 1e-300 + 1e-300;
   const double eps = 2.220446049250313e-16;
@@ -963,9 +981,9 @@ __device__ __forceinline__ void tridiag_lowest_wave(TriLds& t, const double* __r
     if ((n - 1) / 64 == c) zl = lane_val(z[c], (n - 1) % 64);
   }
   if (lane == 0) {
-    st[0] = theta;
+    st[0] = ldexp(theta, ex);
     st[1] = has_bres ? fabs(bres_v * zl * sg) : 0.0;
-    st[2] = tnorm;
+    st[2] = ldexp(tnorm, ex);
   }
 #pragma unroll
   for (int c = 0; c < NC; ++c)
@@ -1125,9 +1143,155 @@ static int finish_step(VT* V, int64_t N, int J, const double* w, const double* p
 
 // ---------------------------------------------------------------------------
 // Dense symmetric tridiagonalisation (one workgroup) and back-transform.
-// A: n x n symmetric in global workspace (overwritten), n <= 256.
 // Householder reflectors H_k = I - tau_k v_k v_k^T act on indices k+1..n-1.
 // ---------------------------------------------------------------------------
+// Lanes a DPP control selects, added (both halves of a double).
+template <int CTRL>
+__device__ __forceinline__ double dpp_add(double x) {
+  const long long u = __double_as_longlong(x);
+  const unsigned lo = __builtin_amdgcn_update_dpp(0, (int)u, CTRL, 0xf, 0xf, true);
+  const unsigned hi = __builtin_amdgcn_update_dpp(0, (int)(u >> 32), CTRL, 0xf, 0xf, true);
+  return x + __longlong_as_double((long long)((unsigned long long)hi << 32 | lo));
+}
+
+// Sum over each group of 16 lanes, in all of them: neighbours, pairs, then
+// the mirrored halves.
+__device__ __forceinline__ double sum16(double x) {
+  x = dpp_add<0xB1>(x);   // quad_perm 1 0 3 2
+  x = dpp_add<0x4E>(x);   // quad_perm 2 3 0 1
+  x = dpp_add<0x141>(x);  // row_half_mirror
+  return dpp_add<0x140>(x);  // row_mirror
+}
+
+__device__ __forceinline__ double sum64(double x) {
+  x = sum16(x);
+  return (lane_val(x, 0) + lane_val(x, 16)) + (lane_val(x, 32) + lane_val(x, 48));
+}
+
+// Tridiagonalisation with the matrix in registers: 16 lanes hold R rows, C
+// elements of each (in pairs of columns), so a step is two barriers: the
+// product p = tau A v with v from LDS (sums inside the 16 lanes), and the
+// rank-2 update with w = p - (tau p.v / 2) v, after which the 16 lanes of the
+// next row form the next reflector alone. M (stride sM between problems) is
+// read once and left as it is. Bound by the latency of those steps: at n = 64 and
+// 128 64 and 205 us, where a thread per row, its row read from L2, took 620 and
+// 2490; at n = 192 1860 against 6000.
+template <int R, int C, int NG>
+__global__ __launch_bounds__(16 * NG) void sytrd_reg_kernel(const double* __restrict__ M, int64_t sM, int n,
+                                                            double* __restrict__ Vst, double* __restrict__ tau,
+                                                            double* __restrict__ dg, double* __restrict__ eg,
+                                                            PMap pm) {
+  {
+    const int64_t o = pm.off();
+    Vst += o; tau += o; dg += o; eg += o;
+    M += (int64_t)pm.pid() * sM;
+  }
+  constexpr int NR = 16 * C;
+  static_assert(R * NG == NR && NG <= 64 && C % 2 == 0, "square, one partial per lane, columns in pairs");
+  __shared__ __attribute__((aligned(16))) double v[NR], p[NR];
+  __shared__ double part[NG], tks;
+  const int t = threadIdx.x, lane = t & 63, s = t & 15, g = t >> 4;
+  auto col = [&](int c) { return 2 * (s + 16 * (c >> 1)) + (c & 1); };
+  double a[R][C];
+#pragma unroll
+  for (int r = 0; r < R; ++r)
+#pragma unroll
+    for (int c = 0; c < C; ++c) {
+      const int i = R * g + r, j = col(c);
+      a[r][c] = i < n && j < n ? M[(int64_t)i * n + j] : 0.0;
+    }
+  // the reflector of row k, by the 16 lanes that hold it
+  auto reflect = [&](int k) {
+    double x[C], sig = 0.0, al = 0.0;
+    const int rk = k % R;
+#pragma unroll
+    for (int c = 0; c < C; ++c) {
+      x[c] = a[0][c];
+#pragma unroll
+      for (int r = 1; r < R; ++r) x[c] = rk == r ? a[r][c] : x[c];
+      const int j = col(c);
+      sig = fma(j > k + 1 ? x[c] : 0.0, x[c], sig);
+      al += j == k + 1 ? x[c] : 0.0;
+    }
+    sig = sum16(sig);
+    al = sum16(al);
+    double tk = 0.0, beta = al, sc = 0.0;
+    if (sig != 0.0) {
+      const double n2 = fma(al, al, sig), rs = rsqrt_nr(n2), nrm = n2 * rs;
+      beta = al >= 0.0 ? -nrm : nrm;
+      tk = fma(fabs(al), rs, 1.0);  // (beta - al) / beta
+      sc = rcp_nr(al - beta);
+    }
+#pragma unroll
+    for (int c = 0; c < C; ++c) {
+      const int j = col(c);
+      const double y = j <= k ? 0.0 : (j == k + 1 ? 1.0 : x[c] * sc);
+      v[j] = y;
+      if (j > k && j < n) Vst[(int64_t)k * n + j - k - 1] = y;
+    }
+    if (s == 0) {
+      tau[k] = tk;
+      eg[k] = beta;
+      tks = tk;
+    }
+  };
+  for (int i = t; i < NR; i += 16 * NG) v[i] = 0.0;
+  __syncthreads();
+  if (g == 0 && n > 2) reflect(0);
+  __syncthreads();
+  for (int k = 0; k + 2 < n; ++k) {
+    const double tk = tks;
+    double vj[C], vi[R], pi[R], pv = 0.0;
+#pragma unroll
+    for (int c = 0; c < C; ++c) vj[c] = v[col(c)];
+#pragma unroll
+    for (int r = 0; r < R; ++r) vi[r] = v[R * g + r];
+#pragma unroll
+    for (int r = 0; r < R; ++r) {
+      double e = 0.0, f = 0.0;
+#pragma unroll
+      for (int c = 0; c < C; c += 2) {
+        e = fma(a[r][c], vj[c], e);
+        f = fma(a[r][c + 1], vj[c + 1], f);
+      }
+      pi[r] = e + f;
+    }
+#pragma unroll
+    for (int r = 0; r < R; ++r) {
+      pi[r] = R * g + r > k ? tk * sum16(pi[r]) : 0.0;
+      pv = fma(pi[r], vi[r], pv);
+    }
+    if (s == 0) {
+#pragma unroll
+      for (int r = 0; r < R; ++r) p[R * g + r] = pi[r];
+      part[g] = pv;
+    }
+    __syncthreads();
+    const double K = 0.5 * tk * sum64(lane < NG ? part[lane] : 0.0);
+    double wj[C];
+#pragma unroll
+    for (int c = 0; c < C; ++c) wj[c] = fma(-K, vj[c], p[col(c)]);
+#pragma unroll
+    for (int r = 0; r < R; ++r) {
+      const double wi = fma(-K, vi[r], pi[r]);
+#pragma unroll
+      for (int c = 0; c < C; ++c) a[r][c] = fma(-vi[r], wj[c], fma(-wi, vj[c], a[r][c]));
+    }
+    if (k + 3 < n && g == (k + 1) / R) reflect(k + 1);
+    __syncthreads();
+  }
+#pragma unroll
+  for (int r = 0; r < R; ++r)
+#pragma unroll
+    for (int c = 0; c < C; ++c) {
+      const int i = R * g + r, j = col(c);
+      if (i == j && i < n) dg[i] = a[r][c];
+      if (i == n - 1 && j == n - 2) eg[n - 2] = a[r][c];
+    }
+}
+
+// The same for 192 < n <= 256: A (n x n, global, overwritten) does not fit in
+// one workgroup's registers.
 __device__ double block_sum(double v, double* red) {
   const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
   v = wave_sum(v);
@@ -1201,31 +1365,97 @@ __global__ __launch_bounds__(256) void sytrd_kernel(double* __restrict__ A, int 
   if (t == 0 && n >= 2) eg[n - 2] = A[(int64_t)(n - 1) * n + (n - 2)];
 }
 
-__global__ __launch_bounds__(256) void ormtr_kernel(const double* __restrict__ Vst,
-                                                   const double* __restrict__ tau, int n,
-                                                   const double* __restrict__ zin,
-                                                   double* __restrict__ x, PMap pm, int64_t so) {
+// x = H_0 H_1 ... H_(n-3) z by one wave, Q elements per lane; the reflectors
+// are read four steps ahead (n = 64, 128: 53, 105 us with two block sums a step,
+// 12, 27 so).
+template <int Q>
+__global__ __launch_bounds__(64) void ormtr_kernel(const double* __restrict__ Vst, const double* __restrict__ tau,
+                                                   int n, const double* __restrict__ zin, double* __restrict__ x,
+                                                   PMap pm, int64_t so) {
   {
     const int64_t o = pm.off();
     Vst += o; tau += o; zin += o;
     x += (int64_t)pm.pid() * so;
   }
-  __shared__ double xs[kTriMax];
-  __shared__ double red[8];
   const int t = threadIdx.x;
-  for (int i = t; i < n; i += blockDim.x) xs[i] = zin[i];
-  __syncthreads();
-  for (int k = n - 3; k >= 0; --k) {
-    const double tk = tau[k];
-    if (tk == 0.0) continue;
-    const int m = n - k - 1;
-    double part = 0.0;
-    for (int i = t; i < m; i += blockDim.x) part += Vst[(int64_t)k * n + i] * xs[k + 1 + i];
-    const double dot = block_sum(part, red);
-    for (int i = t; i < m; i += blockDim.x) xs[k + 1 + i] -= tk * Vst[(int64_t)k * n + i] * dot;
-    __syncthreads();
+  double xs[Q];
+#pragma unroll
+  for (int q = 0; q < Q; ++q) xs[q] = t + 64 * q < n ? zin[t + 64 * q] : 0.0;
+  double v[4][Q], tk[4];
+  auto load = [&](int k0) {
+#pragma unroll
+    for (int u = 0; u < 4; ++u) {
+      const int k = k0 - u;
+      tk[u] = k >= 0 ? tau[k] : 0.0;
+#pragma unroll
+      for (int q = 0; q < Q; ++q) {
+        const int i = t + 64 * q;
+        v[u][q] = k >= 0 && i > k && i < n ? Vst[(int64_t)k * n + i - k - 1] : 0.0;
+      }
+    }
+  };
+  load(n - 3);
+  for (int k = n - 3; k >= 0; k -= 4) {
+    double w[4][Q], f[4];
+#pragma unroll
+    for (int u = 0; u < 4; ++u) {
+      f[u] = tk[u];
+#pragma unroll
+      for (int q = 0; q < Q; ++q) w[u][q] = v[u][q];
+    }
+    load(k - 4);
+#pragma unroll
+    for (int u = 0; u < 4; ++u) {
+      double d = 0.0;
+#pragma unroll
+      for (int q = 0; q < Q; ++q) d = fma(w[u][q], xs[q], d);
+      d = -f[u] * sum64(d);
+#pragma unroll
+      for (int q = 0; q < Q; ++q) xs[q] = fma(d, w[u][q], xs[q]);
+    }
   }
-  for (int i = t; i < n; i += blockDim.x) x[i] = xs[i];
+#pragma unroll
+  for (int q = 0; q < Q; ++q)
+    if (t + 64 * q < n) x[t + 64 * q] = xs[q];
+}
+
+// Tridiagonal form of `batch` matrices M (stride sM between them) by the form
+// that holds them in registers; A is workspace for those that do not fit.
+static int sytrd(const double* M, int64_t sM, int n, double* A, double* Vst, double* tau, double* dg, double* eg,
+                 int batch, PMap pm, hipStream_t s) {
+#define TNX_SYTRD(R_, C_, NG_)                                                                                     \
+  hipLaunchKernelGGL((sytrd_reg_kernel<R_, C_, NG_>), dim3(1, batch), dim3(16 * NG_), 0, s, M, sM, n, Vst, tau, dg, \
+                     eg, pm)
+  if (n <= 32) {
+    TNX_SYTRD(2, 2, 16);
+  } else if (n <= 64) {
+    TNX_SYTRD(2, 4, 32);
+  } else if (n <= 128) {
+    TNX_SYTRD(2, 8, 64);
+  } else if (n <= 192) {
+    TNX_SYTRD(6, 12, 32);
+  } else {
+    const int64_t nn = (int64_t)n * n;
+    hipLaunchKernelGGL(copy_map_kernel, dim3(vec_blocks(nn, batch), batch), dim3(256), 0, s, M, A, nn, pm, sM,
+                       pm.sp);
+    TNX_LAUNCH_CHECK();
+    hipLaunchKernelGGL(sytrd_kernel, dim3(1, batch), dim3(256), 0, s, A, n, Vst, tau, dg, eg, pm);
+  }
+#undef TNX_SYTRD
+  TNX_LAUNCH_CHECK();
+  return TNX_OK;
+}
+
+static int ormtr(const double* Vst, const double* tau, int n, const double* z, double* x, int batch, PMap pm,
+                 int64_t so, hipStream_t s) {
+  if (n <= 64)
+    hipLaunchKernelGGL(ormtr_kernel<1>, dim3(1, batch), dim3(64), 0, s, Vst, tau, n, z, x, pm, so);
+  else if (n <= 128)
+    hipLaunchKernelGGL(ormtr_kernel<2>, dim3(1, batch), dim3(64), 0, s, Vst, tau, n, z, x, pm, so);
+  else
+    hipLaunchKernelGGL(ormtr_kernel<4>, dim3(1, batch), dim3(64), 0, s, Vst, tau, n, z, x, pm, so);
+  TNX_LAUNCH_CHECK();
+  return TNX_OK;
 }
 
 size_t syev_ws_bytes(int n) {
@@ -1247,7 +1477,6 @@ int syev_lowest(const double* M, int n, double* evec, double* eval_host, void* w
   double* eg = dg + n;
   double* z = eg + n;
   double* st = z + n + 8;
-  TNX_HIP(hipMemcpyAsync(A, M, sizeof(double) * n * n, hipMemcpyDeviceToDevice, s));
   if (n == 1) {
     TNX_TRY(fill_f64(evec, 1, 1.0, s));
     if (eval_host) {
@@ -1256,13 +1485,10 @@ int syev_lowest(const double* M, int n, double* evec, double* eval_host, void* w
     }
     return TNX_OK;
   }
-  hipLaunchKernelGGL(sytrd_kernel, dim3(1), dim3(256), 0, s, A, n, Vst, tau, dg, eg, kOne);
-  TNX_LAUNCH_CHECK();
+  TNX_TRY(sytrd(M, 0, n, A, Vst, tau, dg, eg, 1, kOne, s));
   hipLaunchKernelGGL(tridiag_lowest_kernel, dim3(1), dim3(64), 0, s, dg, eg, n, z, st, kOne);
   TNX_LAUNCH_CHECK();
-  hipLaunchKernelGGL(ormtr_kernel, dim3(1), dim3(256), 0, s, Vst, tau, n, z, evec, kOne,
-                     (int64_t)0);
-  TNX_LAUNCH_CHECK();
+  TNX_TRY(ormtr(Vst, tau, n, z, evec, 1, kOne, 0, s));
   if (eval_host) {
     TNX_HIP(hipMemcpyAsync(eval_host, st, sizeof(double), hipMemcpyDeviceToHost, s));
     TNX_HIP(hipStreamSynchronize(s));
@@ -1797,13 +2023,10 @@ static int gd_correction(EigCtx& c, const float* V32, int J32, int keep, int m, 
       TNX_TRY(fill_f64(k.s, 1, 1.0, s));
       TNX_HIP(hipMemcpyAsync(stg, A, sizeof(double), hipMemcpyDeviceToDevice, s));
     } else {
-      hipLaunchKernelGGL(sytrd_kernel, dim3(1), dim3(256), 0, s, A, J, Vst, tau, dg, eg, kOne);
-      TNX_LAUNCH_CHECK();
+      TNX_TRY(sytrd(A, 0, J, nullptr, Vst, tau, dg, eg, 1, kOne, s));  // J <= 64
       hipLaunchKernelGGL(tridiag_lowest_kernel, dim3(1), dim3(64), 0, s, dg, eg, J, zt, stg, kOne);
       TNX_LAUNCH_CHECK();
-      hipLaunchKernelGGL(ormtr_kernel, dim3(1), dim3(256), 0, s, Vst, tau, J, zt, k.s, kOne,
-                         (int64_t)0);
-      TNX_LAUNCH_CHECK();
+      TNX_TRY(ormtr(Vst, tau, J, zt, k.s, 1, kOne, 0, s));
     }
     // z = V s -> k.y, H z = W s -> k.w, r -> V[J] (the next basis slot)
     double* r = V + (int64_t)J * N;
@@ -2589,16 +2812,10 @@ int syev_lowest_b(const double* M, int n, int batch, double* evec, double* eval_
   double* z = eg + n;
   double* st = z + n + 8;
   const PMap pm{nullptr, sp};
-  hipLaunchKernelGGL(copy_map_kernel, dim3(vec_blocks(nn, batch), batch), dim3(256), 0, s, M, A,
-                     nn, pm, nn, sp);
-  TNX_LAUNCH_CHECK();
-  hipLaunchKernelGGL(sytrd_kernel, dim3(1, batch), dim3(256), 0, s, A, n, Vst, tau, dg, eg, pm);
-  TNX_LAUNCH_CHECK();
+  TNX_TRY(sytrd(M, nn, n, A, Vst, tau, dg, eg, batch, pm, s));
   hipLaunchKernelGGL(tridiag_lowest_kernel, dim3(1, batch), dim3(64), 0, s, dg, eg, n, z, st, pm);
   TNX_LAUNCH_CHECK();
-  hipLaunchKernelGGL(ormtr_kernel, dim3(1, batch), dim3(256), 0, s, Vst, tau, n, z, evec, pm,
-                     (int64_t)n);
-  TNX_LAUNCH_CHECK();
+  TNX_TRY(ormtr(Vst, tau, n, z, evec, batch, pm, n, s));
   hipLaunchKernelGGL(gather_status_kernel, dim3(1, batch), dim3(64), 0, s, st, 0, 1, ev, pm);
   TNX_LAUNCH_CHECK();
   TNX_HIP(hipMemcpyAsync(eval_host, ev, sizeof(double) * batch, hipMemcpyDeviceToHost, s));
