@@ -6,7 +6,7 @@
 //
 // Algorithm (a >= b shown; a < b first reduces X to the square R0^T of
 // X^T = Q0 R0):
-//   1. X = Q1 R1 (Householder QR, b x b R1),
+//   1. X = Q1 R1 (b x b R1),
 //   2. R1^T = Q2 R2 (a second QR step: R2 is close to diagonal in the graded
 //      sense, which cuts the Jacobi sweeps from 15..35 to 6..8 on decaying
 //      spectra),
@@ -17,13 +17,14 @@
 //      two blocks of a pair are adjacent after a fixed permutation of block
 //      positions applied between rounds. Per round: the Gram matrices of
 //      all pairs (one batched GEMM), one sweep of two-sided cyclic Jacobi
-//      on each 2kJw x 2kJw Gram matrix in LDS (its rotations kept as Z),
+//      on each 2kJw x 2kJw Gram matrix (its rotations kept as Z; after a
+//      sweep's first round only the pairs across the two blocks),
 //      the rows rotated (P <- Z^T P, one batched GEMM), then the positions
 //      permuted. Rotation angles are the small ones (|theta| <= pi/4), so a
 //      pair that is already orthogonal gets Z ~ I and rows keep their
 //      blocks (sorting them would stall the tournament),
 //   4. singular values = row norms, sorted; W_k = the top-k normalised
-//      rows, made exactly orthonormal by a Householder QR of W_k^T;
+//      rows, made exactly orthonormal by a QR of W_k^T;
 //      U_k = Q1 W_k and U_k^T X = W_k^T R1.
 // Convergence: every pair's off-diagonal |G_ij| <= tol * max(sqrt(G_ii
 // G_jj), floor), checked once per sweep (one host read).
@@ -42,7 +43,6 @@ size_t qr_ws_bytes(int m, int n);
 
 constexpr int kJw = 32;           // rows per Jacobi block
 constexpr int kJp = 2 * kJw;      // rows of a block pair
-constexpr int kJld = kJp + 1;     // LDS row stride
 constexpr int kJacMaxSweeps = 30;
 constexpr double kJacTol = 1e-14;   // relative orthogonality of a row pair
 constexpr double kJacFloor = 1e-28; // times ||X||_F^2: rows below ~1e-14 s_max
@@ -50,115 +50,192 @@ constexpr double kJacFloor = 1e-28; // times ||X||_F^2: rows below ~1e-14 s_max
 
 static size_t al(size_t x) { return (x + 255) & ~(size_t)255; }
 
-// One sweep of two-sided cyclic Jacobi (round-robin, kJp - 1 rounds of kJw
-// disjoint rotations) on each pair's Gram matrix G (kJp x kJp, row-major);
-// Z accumulates the rotations (G_final = Z^T G Z). A round's kJw rotations
-// partition the kJp indices, so G <- J^T G J is one pass over 2 x 2 blocks
-// (rows {p_k, q_k}, columns {p_l, q_l} of rotations k and l) with no two
-// threads touching one entry, and Z <- Z J one pass over row pairs: two
-// barriers per round. Also the pair's off-diagonal measure, max-reduced
-// into *off_bits (a non-negative double read as an unsigned integer, so
-// integer max = double max).
-__global__ __launch_bounds__(256) void jacobi_pair_kernel(const double* __restrict__ Gall,
+typedef double jac_f64x2 __attribute__((ext_vector_type(2)));
+typedef double jac_f64x4 __attribute__((ext_vector_type(4)));
+
+template <int CTRL>
+__device__ __forceinline__ double jac_dpp(double x) {
+  const long long u = __double_as_longlong(x);
+  const unsigned lo = __builtin_amdgcn_update_dpp(0, (int)u, CTRL, 0xf, 0xf, true);
+  const unsigned hi = __builtin_amdgcn_update_dpp(0, (int)(u >> 32), CTRL, 0xf, 0xf, true);
+  return __longlong_as_double((long long)((unsigned long long)hi << 32 | lo));
+}
+
+// One sweep of two-sided cyclic Jacobi on each pair's Gram matrix G (kJp x
+// kJp, row-major); Z accumulates the rotations (G_final = Z^T G Z). Rotation l
+// of a round takes places e_l and o_l (rows l and kJw + l at the start), and
+// after it the rows move on: in a full sweep (kJp - 1 rounds, every pair
+// once) by the round-robin tournament, e_0 fixed; with `cross` (kJw rounds,
+// the pairs of a row of one block with one of the other) o_l takes o_(l+1).
+// Both are back in place after the last round. Also the pair's off-diagonal
+// measure, max-reduced into *off_bits (a non-negative double read as an
+// unsigned integer, so integer max = double max).
+//
+// Everything stays in registers. Threads 0..255, in 16 x 16, hold 4 x 4
+// entries of G each (two rotations' rows and columns): the 16 with a diagonal
+// block find the angles; rows move between threads through LDS, columns
+// between neighbouring lanes. Threads 256..511 hold 16 entries of a row of Z
+// (four lanes a row). Bound by the chain angle - rotation - move, two barriers
+// a round. At 64 x 64, 63 rounds, with G and Z in LDS and the rotations
+// addressed by index 98 us.
+__global__ __launch_bounds__(512) void jacobi_pair_kernel(const double* __restrict__ Gall,
                                                          double* __restrict__ Zall,
-                                                         const double* __restrict__ floor2,
+                                                         const double* __restrict__ floor2, int cross,
                                                          unsigned long long* __restrict__ off_bits) {
-  __shared__ double G[kJp * kJld];
-  __shared__ double Z[kJp * kJld];
-  __shared__ double cs[kJw], sn[kJw];
-  __shared__ int pp[kJw], qq[kJw];
-  __shared__ double red[4];
+  __shared__ __attribute__((aligned(32))) jac_f64x4 xe[256], xo[256];  // rows on their way
+  __shared__ __attribute__((aligned(16))) jac_f64x2 cs[2][kJw];
+  __shared__ double dg[kJp], red[4];
   const int tid = threadIdx.x;
+  const bool inz = tid >= 256;
+  const int tx = tid & 15, ty = (tid >> 4) & 15;      // of G
+  const int zr = (tid & 255) >> 2, zq = tid & 3;      // row and quarter of Z
   const double* Gp = Gall + (size_t)blockIdx.x * kJp * kJp;
-  for (int e = tid; e < kJp * kJp; e += 256) {
-    const int i = e >> 6, j = e & (kJp - 1);
-    // symmetrise (the GEMM's two halves round independently)
-    G[i * kJld + j] = 0.5 * (Gp[e] + Gp[j * kJp + i]);
-    Z[i * kJld + j] = i == j ? 1.0 : 0.0;
-  }
-  __syncthreads();
-  // off-diagonal measure of the incoming pair
-  {
-    const double fl = floor2[0];
-    double mx = 0.0;
-    for (int e = tid; e < kJp * kJp; e += 256) {
-      const int i = e >> 6, j = e & (kJp - 1);
-      if (i != j) {
-        const double den = fmax(sqrt(fmax(G[i * kJld + i], 0.0) * fmax(G[j * kJld + j], 0.0)), fl);
-        mx = fmax(mx, fabs(G[i * kJld + j]) / den);
+  auto place = [](int pair, int h) { return pair + kJw * h; };
+  // x[r][c]: row pair 2 ty + r / 2, column pair 2 tx + c / 2 (h = r % 2, c % 2)
+  // of G; for Z x[i / 4][i % 4] is pair 8 zq + i / 2, h = i % 2
+  double x[4][4];
+#pragma unroll
+  for (int r = 0; r < 4; ++r)
+#pragma unroll
+    for (int c = 0; c < 4; ++c) {
+      if (inz) {
+        const int i = 4 * r + c;
+        x[r][c] = place(8 * zq + (i >> 1), i & 1) == zr ? 1.0 : 0.0;
+      } else {
+        // symmetrise (the GEMM's two halves round independently)
+        const int i = place(2 * ty + (r >> 1), r & 1), j = place(2 * tx + (c >> 1), c & 1);
+        x[r][c] = 0.5 * (Gp[i * kJp + j] + Gp[j * kJp + i]);
       }
     }
+  // ---- off-diagonal measure of the incoming pair: |G_ij| over the larger of
+  // sqrt(G_ii G_jj) and the floor
+  if (!inz && tx == ty) {
+#pragma unroll
+    for (int r = 0; r < 4; ++r) dg[place(2 * ty + (r >> 1), r & 1)] = rsqrt_nr(fmax(x[r][r], 1e-300));
+  }
+  __syncthreads();
+  if (!inz) {
+    const double ifl = 1.0 / floor2[0];
+    double mx = 0.0;
+#pragma unroll
+    for (int r = 0; r < 4; ++r)
+#pragma unroll
+      for (int c = 0; c < 4; ++c) {
+        const int i = place(2 * ty + (r >> 1), r & 1), j = place(2 * tx + (c >> 1), c & 1);
+        const double o = fabs(x[r][c]) * fmin(dg[i] * dg[j], ifl);
+        mx = i != j ? fmax(mx, o) : mx;
+      }
 #pragma unroll
     for (int o = 32; o > 0; o >>= 1) mx = fmax(mx, __shfl_xor(mx, o, 64));
     if ((tid & 63) == 0) red[tid >> 6] = mx;
-    __syncthreads();
-    if (tid == 0) {
-      const double m = fmax(fmax(red[0], red[1]), fmax(red[2], red[3]));
-      atomicMax(off_bits, (unsigned long long)__double_as_longlong(m));
-    }
   }
-  for (int r = 0; r < kJp - 1; ++r) {
-    if (tid < kJw) {
-      const int i = tid;
-      int p, q;
-      if (i == 0) {
-        p = 0;
-        q = 1 + ((kJp - 2 - r) % (kJp - 1) + (kJp - 1)) % (kJp - 1);
-      } else {
-        p = 1 + ((i - 1 - r) % (kJp - 1) + (kJp - 1)) % (kJp - 1);
-        q = 1 + ((kJp - 2 - i - r) % (kJp - 1) + (kJp - 1)) % (kJp - 1);
-      }
-      const double a = G[p * kJld + p], d = G[q * kJld + q], b = G[p * kJld + q];
-      double c = 1.0, s = 0.0;
-      if (b != 0.0) {
+  __syncthreads();
+  if (tid == 0)
+    atomicMax(off_bits,
+              (unsigned long long)__double_as_longlong(fmax(fmax(red[0], red[1]), fmax(red[2], red[3]))));
+  const int rounds = cross ? kJw : kJp - 1;
+  for (int r = 0; r < rounds; ++r) {
+    jac_f64x2* w = cs[r & 1];
+    if (!inz && tx == ty) {
+#pragma unroll
+      for (int k = 0; k < 2; ++k) {
+        const double a = x[2 * k][2 * k], d = x[2 * k + 1][2 * k + 1], b = x[2 * k][2 * k + 1];
         // t = sign(zeta) / (|zeta| + sqrt(1 + zeta^2)), zeta = (d - a) / (2 b);
-        // the refined reciprocals only see arguments >= 1
-        const double zeta = (d - a) / (2.0 * b);
-        double t;
-        if (fabs(zeta) > 1e100) {
-          t = 0.5 / zeta;
-        } else {
-          const double w = fma(zeta, zeta, 1.0);
-          t = (zeta >= 0.0 ? 1.0 : -1.0) * rcp_nr(fabs(zeta) + w * rsqrt_nr(w));
-        }
-        c = rsqrt_nr(fma(t, t, 1.0));
-        s = c * t;
+        // nothing to do for a negligible b
+        const double zeta = (d - a) * rcp_nr(2.0 * b), u = fma(zeta, zeta, 1.0);
+        const double q = rcp_nr(fabs(zeta) + u * rsqrt_nr(u)), t = zeta >= 0.0 ? q : -q;
+        const double c = rsqrt_nr(fma(t, t, 1.0));
+        const bool on = b != 0.0 && fabs(zeta) < 1e100;
+        w[2 * ty + k] = jac_f64x2{on ? c : 1.0, on ? c * t : 0.0};
       }
-      cs[i] = c; sn[i] = s; pp[i] = p; qq[i] = q;
     }
     __syncthreads();
-    // G <- J^T G J, one 2 x 2 block per (k, l)
-    for (int e = tid; e < kJw * kJw; e += 256) {
-      const int k = e >> 5, l = e & (kJw - 1);
-      const int pk = pp[k], qk = qq[k], pl = pp[l], ql = qq[l];
-      const double ck = cs[k], sk = sn[k], cl = cs[l], sl = sn[l];
-      const double g00 = G[pk * kJld + pl], g01 = G[pk * kJld + ql];
-      const double g10 = G[qk * kJld + pl], g11 = G[qk * kJld + ql];
-      // rows: [r0; r1] = J_k^T [g0; g1]
-      const double r00 = ck * g00 - sk * g10, r01 = ck * g01 - sk * g11;
-      const double r10 = sk * g00 + ck * g10, r11 = sk * g01 + ck * g11;
-      // columns: [c0 c1] = [r0 r1] J_l
-      G[pk * kJld + pl] = cl * r00 - sl * r01;
-      G[pk * kJld + ql] = sl * r00 + cl * r01;
-      G[qk * kJld + pl] = cl * r10 - sl * r11;
-      G[qk * kJld + ql] = sl * r10 + cl * r11;
+    if (inz) {
+      // Z <- Z J, then the columns move on
+      double* z = &x[0][0];
+#pragma unroll
+      for (int l = 0; l < 8; ++l) {
+        const jac_f64x2 v = w[8 * zq + l];
+        const double e = z[2 * l], o = z[2 * l + 1];
+        z[2 * l] = v[0] * e - v[1] * o;
+        z[2 * l + 1] = v[1] * e + v[0] * o;
+      }
+      const double ei = jac_dpp<0x90>(z[14]);  // quad_perm 0 0 1 2: from the quarter before
+      const double oi = jac_dpp<0x39>(z[1]);   // quad_perm 1 2 3 0: from the quarter behind
+      const double e0 = z[0], o0 = z[1], e7 = z[14];
+#pragma unroll
+      for (int l = 0; l < 7; ++l) z[2 * l + 1] = z[2 * l + 3];
+      z[15] = zq == 3 && !cross ? e7 : oi;
+      if (!cross) {
+#pragma unroll
+        for (int l = 7; l > 1; --l) z[2 * l] = z[2 * l - 2];
+        z[2] = zq == 0 ? o0 : e0;
+        z[0] = zq == 0 ? e0 : ei;
+      }
+      __syncthreads();
+      continue;
     }
-    // Z <- Z J
-    for (int e = tid; e < kJp * kJw; e += 256) {
-      const int j = e >> 5, l = e & (kJw - 1);
-      const int pl = pp[l], ql = qq[l];
-      const double cl = cs[l], sl = sn[l];
-      const double zp = Z[j * kJld + pl], zq = Z[j * kJld + ql];
-      Z[j * kJld + pl] = cl * zp - sl * zq;
-      Z[j * kJld + ql] = sl * zp + cl * zq;
+    const jac_f64x2 k0 = w[2 * ty], k1 = w[2 * ty + 1], l0 = w[2 * tx], l1 = w[2 * tx + 1];
+#pragma unroll
+    for (int k = 0; k < 2; ++k) {
+      const double c = k ? k1[0] : k0[0], sn = k ? k1[1] : k0[1];
+#pragma unroll
+      for (int j = 0; j < 4; ++j) {
+        const double e = x[2 * k][j], o = x[2 * k + 1][j];
+        x[2 * k][j] = c * e - sn * o;
+        x[2 * k + 1][j] = sn * e + c * o;
+      }
     }
+#pragma unroll
+    for (int l = 0; l < 2; ++l) {
+      const double c = l ? l1[0] : l0[0], sn = l ? l1[1] : l0[1];
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        const double e = x[i][2 * l], o = x[i][2 * l + 1];
+        x[i][2 * l] = c * e - sn * o;
+        x[i][2 * l + 1] = sn * e + c * o;
+      }
+    }
+    // columns move between the 16 lanes of a row of threads
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      const double e0 = x[i][0], o0 = x[i][1], e1 = x[i][2], o1 = x[i][3];
+      const double oi = jac_dpp<0x12F>(o0);  // row_ror:15, from the lane behind
+      x[i][1] = o1;
+      x[i][3] = tx == 15 && !cross ? e1 : oi;
+      if (!cross) {
+        const double ei = jac_dpp<0x121>(e1);  // row_ror:1, from the lane before
+        x[i][0] = tx == 0 ? e0 : ei;
+        x[i][2] = tx == 0 ? o0 : e0;
+      }
+    }
+    // rows move between rows of threads
+    xo[tid] = jac_f64x4{x[1][0], x[1][1], x[1][2], x[1][3]};
+    if (!cross) xe[tid] = jac_f64x4{x[2][0], x[2][1], x[2][2], x[2][3]};
     __syncthreads();
+    const jac_f64x4 oi = xo[(tid + 16) & 255];
+    jac_f64x4 ei = {0.0, 0.0, 0.0, 0.0};
+    if (!cross) ei = xe[(tid + 240) & 255];
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+      const double e0 = x[0][j], o0 = x[1][j], e1 = x[2][j], o1 = x[3][j];
+      x[1][j] = o1;
+      x[3][j] = ty == 15 && !cross ? e1 : oi[j];
+      if (!cross) {
+        x[0][j] = ty == 0 ? e0 : ei[j];
+        x[2][j] = ty == 0 ? o0 : e0;
+      }
+    }
   }
+  if (!inz) return;
   double* Zp = Zall + (size_t)blockIdx.x * kJp * kJp;
-  for (int e = tid; e < kJp * kJp; e += 256) {
-    const int i = e >> 6, j = e & (kJp - 1);
-    Zp[e] = Z[i * kJld + j];
-  }
+#pragma unroll
+  for (int r = 0; r < 4; ++r)
+#pragma unroll
+    for (int c = 0; c < 4; ++c) {
+      const int i = 4 * r + c;
+      Zp[zr * kJp + place(8 * zq + (i >> 1), i & 1)] = x[r][c];
+    }
 }
 
 __global__ void jacobi_permute_kernel(const double* __restrict__ src, double* __restrict__ dst,
@@ -303,7 +380,8 @@ static int jacobi_rows(const double* X0, int p, int q, void* ws, double** Xout, 
       g.alpha = 1.0; g.beta = 0.0; g.prec = Prec::F64;
       g.splitk_ws = part; g.splitk_ws_bytes = (size_t)8 * npair * kJp * kJp * 8;
       TNX_TRY(gemm(g, s));
-      hipLaunchKernelGGL(jacobi_pair_kernel, dim3(npair), dim3(256), 0, s, G, Z, floor2, off_bits);
+      // a block's own pairs once per sweep, in its first round
+      hipLaunchKernelGGL(jacobi_pair_kernel, dim3(npair), dim3(512), 0, s, G, Z, floor2, r > 0 ? 1 : 0, off_bits);
       TNX_LAUNCH_CHECK();
       // Y_i = Z_i^T P_i
       GemmDesc g2{};
