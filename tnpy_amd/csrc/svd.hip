@@ -65,7 +65,7 @@ __device__ __forceinline__ double jac_dpp(double x) {
 // kJp, row-major); Z accumulates the rotations (G_final = Z^T G Z). Rotation l
 // of a round takes places e_l and o_l (rows l and kJw + l at the start), and
 // after it the rows move on: in a full sweep (kJp - 1 rounds, every pair
-// once) by the round-robin tournament, e_0 fixed; with `cross` (kJw rounds,
+// once) by the round-robin tournament, e_0 fixed; with CROSS (kJw rounds,
 // the pairs of a row of one block with one of the other) o_l takes o_(l+1).
 // Both are back in place after the last round. Also the pair's off-diagonal
 // measure, max-reduced into *off_bits (a non-negative double read as an
@@ -73,14 +73,16 @@ __device__ __forceinline__ double jac_dpp(double x) {
 //
 // Everything stays in registers. Threads 0..255, in 16 x 16, hold 4 x 4
 // entries of G each (two rotations' rows and columns): the 16 with a diagonal
-// block find the angles; rows move between threads through LDS, columns
-// between neighbouring lanes. Threads 256..511 hold 16 entries of a row of Z
+// block and the lanes behind them find the angles; rows move between threads
+// through LDS, columns between neighbouring lanes. Threads 256..511 hold 16 entries of a row of Z
 // (four lanes a row). Bound by the chain angle - rotation - move, two barriers
-// a round. At 64 x 64, 63 rounds, with G and Z in LDS and the rotations
-// addressed by index 98 us.
+// a round: 55 us for the 63 rounds of a full sweep. With G and Z in LDS and the
+// rotations addressed by index 98 us; with correctly rounded angles, both of a
+// block's by its own lane, 90.
+template <bool CROSS>
 __global__ __launch_bounds__(512) void jacobi_pair_kernel(const double* __restrict__ Gall,
                                                          double* __restrict__ Zall,
-                                                         const double* __restrict__ floor2, int cross,
+                                                         const double* __restrict__ floor2,
                                                          unsigned long long* __restrict__ off_bits) {
   __shared__ __attribute__((aligned(32))) jac_f64x4 xe[256], xo[256];  // rows on their way
   __shared__ __attribute__((aligned(16))) jac_f64x2 cs[2][kJw];
@@ -133,77 +135,83 @@ __global__ __launch_bounds__(512) void jacobi_pair_kernel(const double* __restri
   if (tid == 0)
     atomicMax(off_bits,
               (unsigned long long)__double_as_longlong(fmax(fmax(red[0], red[1]), fmax(red[2], red[3]))));
-  const int rounds = cross ? kJw : kJp - 1;
-  for (int r = 0; r < rounds; ++r) {
-    jac_f64x2* w = cs[r & 1];
-    if (!inz && tx == ty) {
-#pragma unroll
-      for (int k = 0; k < 2; ++k) {
-        const double a = x[2 * k][2 * k], d = x[2 * k + 1][2 * k + 1], b = x[2 * k][2 * k + 1];
-        // t = sign(zeta) / (|zeta| + sqrt(1 + zeta^2)), zeta = (d - a) / (2 b);
-        // nothing to do for a negligible b
-        const double zeta = (d - a) * rcp_nr(2.0 * b), u = fma(zeta, zeta, 1.0);
-        const double q = rcp_nr(fabs(zeta) + u * rsqrt_nr(u)), t = zeta >= 0.0 ? q : -q;
-        const double c = rsqrt_nr(fma(t, t, 1.0));
-        const bool on = b != 0.0 && fabs(zeta) < 1e100;
-        w[2 * ty + k] = jac_f64x2{on ? c : 1.0, on ? c * t : 0.0};
-      }
-    }
-    __syncthreads();
-    if (inz) {
+  constexpr int rounds = CROSS ? kJw : kJp - 1;
+  if (inz) {
+    double* z = &x[0][0];
+    for (int r = 0; r < rounds; ++r) {
+      __syncthreads();
       // Z <- Z J, then the columns move on
-      double* z = &x[0][0];
 #pragma unroll
       for (int l = 0; l < 8; ++l) {
-        const jac_f64x2 v = w[8 * zq + l];
+        const jac_f64x2 v = cs[r & 1][8 * zq + l];
         const double e = z[2 * l], o = z[2 * l + 1];
         z[2 * l] = v[0] * e - v[1] * o;
         z[2 * l + 1] = v[1] * e + v[0] * o;
       }
-      const double ei = jac_dpp<0x90>(z[14]);  // quad_perm 0 0 1 2: from the quarter before
-      const double oi = jac_dpp<0x39>(z[1]);   // quad_perm 1 2 3 0: from the quarter behind
+      const double oi = jac_dpp<0x39>(z[1]);  // quad_perm 1 2 3 0: from the quarter behind
       const double e0 = z[0], o0 = z[1], e7 = z[14];
 #pragma unroll
       for (int l = 0; l < 7; ++l) z[2 * l + 1] = z[2 * l + 3];
-      z[15] = zq == 3 && !cross ? e7 : oi;
-      if (!cross) {
+      z[15] = !CROSS && zq == 3 ? e7 : oi;
+      if (!CROSS) {
+        const double ei = jac_dpp<0x90>(e7);  // quad_perm 0 0 1 2: from the quarter before
 #pragma unroll
         for (int l = 7; l > 1; --l) z[2 * l] = z[2 * l - 2];
         z[2] = zq == 0 ? o0 : e0;
         z[0] = zq == 0 ? e0 : ei;
       }
       __syncthreads();
-      continue;
     }
-    const jac_f64x2 k0 = w[2 * ty], k1 = w[2 * ty + 1], l0 = w[2 * tx], l1 = w[2 * tx + 1];
+    double* Zp = Zall + (size_t)blockIdx.x * kJp * kJp;
 #pragma unroll
-    for (int k = 0; k < 2; ++k) {
-      const double c = k ? k1[0] : k0[0], sn = k ? k1[1] : k0[1];
+    for (int i = 0; i < 16; ++i) Zp[zr * kJp + place(8 * zq + (i >> 1), i & 1)] = z[i];
+    return;
+  }
+  // the second rotation of a diagonal block is worked out by the next lane
+  const int own = (tx - ty) & 15;  // 0: the block's lane, 1: the next one
+  for (int r = 0; r < rounds; ++r) {
+    const double a1 = jac_dpp<0x121>(x[2][2]), d1 = jac_dpp<0x121>(x[3][3]), b1 = jac_dpp<0x121>(x[2][3]);
+    if (own < 2) {
+      const double a = own ? a1 : x[0][0], d = own ? d1 : x[1][1], b = own ? b1 : x[0][1];
+      // t = sign(zeta) / (|zeta| + sqrt(1 + zeta^2)), zeta = (d - a) / (2 b);
+      // nothing to do for a negligible b. One Newton step each (1e-8 or better
+      // of the angle, so of b is left for the next sweep); c and s = c t are a
+      // rotation to rounding.
+      const double b2 = 2.0 * b, i0 = __builtin_amdgcn_rcp(b2), i1 = fma(i0, fma(-b2, i0, 1.0), i0);
+      const double zeta = (d - a) * i1, u = fma(zeta, zeta, 1.0);
+      const double q0 = __builtin_amdgcn_rsq(u), q1 = fma(0.5 * q0, fma(-u * q0, q0, 1.0), q0);
+      const double v = fma(u, q1, fabs(zeta)), p0 = __builtin_amdgcn_rcp(v), p1 = fma(p0, fma(-v, p0, 1.0), p0);
+      const double t = zeta >= 0.0 ? p1 : -p1, c = rsqrt_nr(fma(t, t, 1.0));
+      const bool on = b != 0.0 && fabs(zeta) < 1e100;
+      cs[r & 1][2 * ty + own] = jac_f64x2{on ? c : 1.0, on ? c * t : 0.0};
+    }
+    __syncthreads();
+    const jac_f64x2* w = cs[r & 1];
+    const jac_f64x2 kr[2] = {w[2 * ty], w[2 * ty + 1]}, lc[2] = {w[2 * tx], w[2 * tx + 1]};
+#pragma unroll
+    for (int k = 0; k < 2; ++k)
 #pragma unroll
       for (int j = 0; j < 4; ++j) {
         const double e = x[2 * k][j], o = x[2 * k + 1][j];
-        x[2 * k][j] = c * e - sn * o;
-        x[2 * k + 1][j] = sn * e + c * o;
+        x[2 * k][j] = kr[k][0] * e - kr[k][1] * o;
+        x[2 * k + 1][j] = kr[k][1] * e + kr[k][0] * o;
       }
-    }
 #pragma unroll
-    for (int l = 0; l < 2; ++l) {
-      const double c = l ? l1[0] : l0[0], sn = l ? l1[1] : l0[1];
+    for (int l = 0; l < 2; ++l)
 #pragma unroll
       for (int i = 0; i < 4; ++i) {
         const double e = x[i][2 * l], o = x[i][2 * l + 1];
-        x[i][2 * l] = c * e - sn * o;
-        x[i][2 * l + 1] = sn * e + c * o;
+        x[i][2 * l] = lc[l][0] * e - lc[l][1] * o;
+        x[i][2 * l + 1] = lc[l][1] * e + lc[l][0] * o;
       }
-    }
     // columns move between the 16 lanes of a row of threads
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
       const double e0 = x[i][0], o0 = x[i][1], e1 = x[i][2], o1 = x[i][3];
       const double oi = jac_dpp<0x12F>(o0);  // row_ror:15, from the lane behind
       x[i][1] = o1;
-      x[i][3] = tx == 15 && !cross ? e1 : oi;
-      if (!cross) {
+      x[i][3] = !CROSS && tx == 15 ? e1 : oi;
+      if (!CROSS) {
         const double ei = jac_dpp<0x121>(e1);  // row_ror:1, from the lane before
         x[i][0] = tx == 0 ? e0 : ei;
         x[i][2] = tx == 0 ? o0 : e0;
@@ -211,31 +219,22 @@ __global__ __launch_bounds__(512) void jacobi_pair_kernel(const double* __restri
     }
     // rows move between rows of threads
     xo[tid] = jac_f64x4{x[1][0], x[1][1], x[1][2], x[1][3]};
-    if (!cross) xe[tid] = jac_f64x4{x[2][0], x[2][1], x[2][2], x[2][3]};
+    if (!CROSS) xe[tid] = jac_f64x4{x[2][0], x[2][1], x[2][2], x[2][3]};
     __syncthreads();
     const jac_f64x4 oi = xo[(tid + 16) & 255];
     jac_f64x4 ei = {0.0, 0.0, 0.0, 0.0};
-    if (!cross) ei = xe[(tid + 240) & 255];
+    if (!CROSS) ei = xe[(tid + 240) & 255];
 #pragma unroll
     for (int j = 0; j < 4; ++j) {
       const double e0 = x[0][j], o0 = x[1][j], e1 = x[2][j], o1 = x[3][j];
       x[1][j] = o1;
-      x[3][j] = ty == 15 && !cross ? e1 : oi[j];
-      if (!cross) {
+      x[3][j] = !CROSS && ty == 15 ? e1 : oi[j];
+      if (!CROSS) {
         x[0][j] = ty == 0 ? e0 : ei[j];
         x[2][j] = ty == 0 ? o0 : e0;
       }
     }
   }
-  if (!inz) return;
-  double* Zp = Zall + (size_t)blockIdx.x * kJp * kJp;
-#pragma unroll
-  for (int r = 0; r < 4; ++r)
-#pragma unroll
-    for (int c = 0; c < 4; ++c) {
-      const int i = 4 * r + c;
-      Zp[zr * kJp + place(8 * zq + (i >> 1), i & 1)] = x[r][c];
-    }
 }
 
 __global__ void jacobi_permute_kernel(const double* __restrict__ src, double* __restrict__ dst,
@@ -381,7 +380,10 @@ static int jacobi_rows(const double* X0, int p, int q, void* ws, double** Xout, 
       g.splitk_ws = part; g.splitk_ws_bytes = (size_t)8 * npair * kJp * kJp * 8;
       TNX_TRY(gemm(g, s));
       // a block's own pairs once per sweep, in its first round
-      hipLaunchKernelGGL(jacobi_pair_kernel, dim3(npair), dim3(512), 0, s, G, Z, floor2, r > 0 ? 1 : 0, off_bits);
+      if (r == 0)
+        hipLaunchKernelGGL(jacobi_pair_kernel<false>, dim3(npair), dim3(512), 0, s, G, Z, floor2, off_bits);
+      else
+        hipLaunchKernelGGL(jacobi_pair_kernel<true>, dim3(npair), dim3(512), 0, s, G, Z, floor2, off_bits);
       TNX_LAUNCH_CHECK();
       // Y_i = Z_i^T P_i
       GemmDesc g2{};
