@@ -1497,24 +1497,26 @@ int syev_lowest(const double* M, int n, double* evec, double* eval_host, void* w
 }
 
 // ---------------------------------------------------------------------------
-// All eigenpairs of a symmetric tridiagonal matrix (n <= 64): implicit QL
-// with Wilkinson shifts, one wavefront. Every lane runs the same scalar
-// recurrence on the LDS copies of the diagonal / off-diagonal and writes the
-// same values to them, so each lane only ever reads its own writes and the
-// recurrence needs no barrier; lane k owns row k of the eigenvector matrix Z
-// and applies each Givens rotation to it. Eigenvalues ascending to w, eigenvectors as columns
-// of S (row stride ldS). Used at thick restarts, where the projected matrix
-// is tridiagonal.
+// All eigenpairs of a symmetric tridiagonal matrix (n <= 64): eigenvalues
+// ascending to w, eigenvectors as columns of S (row stride ldS). Used at thick
+// restarts, where the projected matrix is tridiagonal.
+//
+// Implicit QL is one chain of about 1.7 n^2 / 2 rotations, 1 ms at n = 64.
+// Instead lane j finds eigenvalue j by sections, four points a round (one per
+// wave, 24 rounds of 1.5 us), and its eigenvector from the twisted
+// factorisation at that value; the vectors, orthonormal to rounding over the
+// relative gap, are then orthonormalised symmetrically (Z <- Z (I - E / 2), E
+// = Z^T Z - I, which converges quadratically and moves each vector least).
+// Mixing two vectors by eps ||T|| / gap changes a residual by eps ||T||, so
+// this is as accurate as QL while E starts small; clusters so tight that it
+// does not (E above 1e-6) take QL.
 // ---------------------------------------------------------------------------
-__global__ __launch_bounds__(64) void tridiag_all_kernel(const double* __restrict__ ad,
-                                                         const double* __restrict__ bd, int n,
-                                                         double* __restrict__ w,
-                                                         double* __restrict__ S, int ldS,
-                                                         PMap pm) {
-  {
-    const int64_t o = pm.off();
-    ad += o; bd += o; w += o; S += o;
-  }
+constexpr int kAllLd = 65;
+typedef double tri_f64x4 __attribute__((ext_vector_type(4)));
+
+// Implicit QL by one wave (threads 0..63); Z: 64 rows of stride kAllLd, dsh: 64.
+__device__ void tridiag_ql_wave(const double* __restrict__ ad, const double* __restrict__ bd, int n,
+                                double* __restrict__ w, double* __restrict__ S, int ldS, double* Z, double* dsh) {
   // Implicit QL with eigenvectors (n <= 64). d[i], e[i] live in lane i's
   // registers: the rotation chain runs on all lanes as wave-uniform scalars,
   // reading a row with v_readlane and writing lane i's value with a lane
@@ -1522,13 +1524,11 @@ __global__ __launch_bounds__(64) void tridiag_all_kernel(const double* __restric
   // private to lane k (in LDS); within a sweep the lane carries the freshly
   // rotated element Z[k][i] in a register to the next step, so its LDS row
   // sees only reads of untouched columns and stores nobody waits for.
-  __shared__ double Z[64][65];
-  __shared__ double dsh[64];
   const int k = threadIdx.x;
   double dr = k < n ? ad[k] : 0.0;
   double er = k < n - 1 ? bd[k] : 0.0;
   if (k < n)
-    for (int c = 0; c < n; ++c) Z[k][c] = (k == c) ? 1.0 : 0.0;
+    for (int c = 0; c < n; ++c) Z[k * kAllLd + c] = (k == c) ? 1.0 : 0.0;
   const double eps = 2.220446049250313e-16;
   for (int l = 0; l < n; ++l) {
     for (int iter = 0; iter < 60; ++iter) {
@@ -1571,30 +1571,210 @@ __global__ __launch_bounds__(64) void tridiag_all_kernel(const double* __restric
         if (k == i + 1) dr = g + p;
         g = cs * r - b;
         if (k < n) {
-          const double zi1 = hidx == i + 1 ? zc : Z[k][i + 1];
-          const double zi = Z[k][i];
-          Z[k][i + 1] = sn * zi + cs * zi1;
+          const double zi1 = hidx == i + 1 ? zc : Z[k * kAllLd + i + 1];
+          const double zi = Z[k * kAllLd + i];
+          Z[k * kAllLd + i + 1] = sn * zi + cs * zi1;
           zc = cs * zi - sn * zi1;
         }
         hidx = i;
       }
       // store the held element: Z[k][l] after a full sweep, Z[k][i+1] when
       // the sweep stopped at step i
-      if (k < n && hidx >= 0) Z[k][hidx] = zc;
+      if (k < n && hidx >= 0) Z[k * kAllLd + hidx] = zc;
       if (early) continue;
       if (k == l) { dr -= p; er = g; }
       if (k == m) er = 0.0;
     }
   }
   if (k < n) dsh[k] = dr;
-  __syncthreads();
+  wave_lds_fence();
   if (k < n) {
     const double dk = dr;
     int rank = 0;
     for (int j = 0; j < n; ++j) rank += (dsh[j] < dk) || (dsh[j] == dk && j < k);
     w[rank] = dk;
-    for (int row = 0; row < n; ++row) S[row * ldS + rank] = Z[row][k];
+    for (int row = 0; row < n; ++row) S[row * ldS + rank] = Z[row * kAllLd + k];
   }
+}
+
+__global__ __launch_bounds__(256) void tridiag_all_kernel(const double* __restrict__ ad,
+                                                          const double* __restrict__ bd, int n,
+                                                          double* __restrict__ w, double* __restrict__ S, int ldS,
+                                                          PMap pm) {
+  {
+    const int64_t o = pm.off();
+    ad += o; bd += o; w += o; S += o;
+  }
+  __shared__ double2 row[kMaxBasis + 16];  // {a_k, b_{k-1}^2}
+  __shared__ double bb[kMaxBasis];         // b_k
+  __shared__ double Z[64 * kAllLd], U[64 * kAllLd], D[64 * kAllLd];
+  __shared__ int cnt[2][4][64];
+  __shared__ double part[2][64], red[4];
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, lr = lane & 15, lk = lane >> 4;
+  // ---- the matrix, by a power of two near 1 where its norm is far from it
+  double a = lane < n ? ad[lane] : 0.0, b = lane < n - 1 ? bd[lane] : 0.0;
+  double bl = lane > 0 && lane < n ? bd[lane - 1] : 0.0;
+  double r0 = fabs(b) + fabs(bl), tn = lane < n ? fabs(a) + r0 : 0.0;
+  for (int o = 32; o > 0; o >>= 1) tn = fmax(tn, __shfl_xor(tn, o, 64));
+  int ex = __builtin_amdgcn_frexp_exp(tn);
+  if (ex >= -64 && ex <= 64) ex = 0;
+  a = ldexp(a, -ex);
+  b = ldexp(b, -ex);
+  bl = ldexp(bl, -ex);
+  r0 = ldexp(r0, -ex);
+  tn = ldexp(tn, -ex);
+  const double eps = 2.220446049250313e-16;
+  double lo = lane < n ? a - r0 : 1e308, hi = lane < n ? a + r0 : -1e308;
+  for (int o = 32; o > 0; o >>= 1) {
+    lo = fmin(lo, __shfl_xor(lo, o, 64));
+    hi = fmax(hi, __shfl_xor(hi, o, 64));
+  }
+  lo -= 4.0 * eps * tn + 1e-300;
+  hi += 4.0 * eps * tn + 1e-300;
+  if (wave == 0) {
+    row[lane] = make_double2(a, bl * bl);
+    bb[lane] = b;
+    if (lane < 16) row[kMaxBasis + lane] = make_double2(0.0, 0.0);
+  }
+  __syncthreads();
+  // ---- eigenvalue `lane`: at most `lane` of them below lo, more below hi;
+  // each round keeps a fifth (5^-24 of the Gershgorin range in the end)
+  const int j = min(lane, n - 1);
+  for (int it = 0; it < 24; ++it) {
+    const double h = 0.2 * (hi - lo), x0 = lo;
+    int c;
+    double g;
+    char_poly(row, n, fma(h, (double)(wave + 1), x0), c, g);
+    cnt[it & 1][wave][lane] = c;
+    __syncthreads();
+    bool found = false;
+#pragma unroll
+    for (int s = 0; s < 4; ++s) {
+      const double x = fma(h, (double)(s + 1), x0);
+      const bool above = cnt[it & 1][s][lane] > j;
+      if (!found) {
+        if (above) hi = x;
+        else lo = x;
+      }
+      found = found || above;
+    }
+  }
+  const double lam = 0.5 * (lo + hi);
+  // ---- twisted factorisation: pivots and their ratios from above (wave 0)
+  // and from below (wave 1)
+  const double tiny = 0.25 * eps * tn + 1e-290;
+  if (wave == 0) {
+    double q = row[0].x - lam;
+    for (int k = 0; k < n; ++k) {
+      if (!(fabs(q) >= tiny)) q = tiny;
+      const double rq = rcp_nr(q);
+      Z[k * kAllLd + lane] = q;
+      U[k * kAllLd + lane] = -bb[k] * rq;
+      q = row[k + 1].x - lam - row[k + 1].y * rq;
+    }
+  } else if (wave == 1) {
+    double q = row[n - 1].x - lam;
+    for (int k = n - 1; k >= 0; --k) {
+      if (!(fabs(q) >= tiny)) q = tiny;
+      const double rq = rcp_nr(q), bk = k > 0 ? bb[k - 1] : 0.0;
+      D[k * kAllLd + lane] = -bk * rq;
+      q = (k > 0 ? row[k - 1].x : 0.0) - lam - bk * bk * rq;
+    }
+  }
+  __syncthreads();
+  // where they meet: the smallest gamma_k = q+_k + b_k D_{k+1}
+  int r = 0;
+  if (wave < 2) {
+    double best = 1e308;
+    for (int k = 0; k < n; ++k) {
+      const double dn = k + 1 < n ? D[(k + 1) * kAllLd + lane] : 0.0;
+      const double gm = fabs(fma(bb[k], dn, Z[k * kAllLd + lane]));
+      r = gm < best ? k : r;
+      best = fmin(best, gm);
+    }
+  }
+  __syncthreads();
+  if (wave < 2) {
+    // z_r = 1, products of ratios upwards (wave 0) and downwards (wave 1)
+    double z = 1.0, nn = 0.0;
+    if (wave == 0) {
+      for (int k = n - 1; k >= 0; --k) {
+        if (k > r) continue;
+        if (k < r) z *= U[k * kAllLd + lane];
+        Z[k * kAllLd + lane] = z;
+        nn = fma(z, z, nn);
+      }
+    } else {
+      for (int k = 1; k < n; ++k) {
+        if (k <= r) continue;
+        z *= D[k * kAllLd + lane];
+        Z[k * kAllLd + lane] = z;
+        nn = fma(z, z, nn);
+      }
+    }
+    part[wave][lane] = nn;
+  }
+  __syncthreads();
+  {
+    const double f = rsqrt_nr(part[0][lane] + part[1][lane]);
+    for (int k = wave; k < 64; k += 4) {
+      const double z = k < n ? Z[k * kAllLd + lane] : 0.0;
+      Z[k * kAllLd + lane] = k < n && lane < n ? z * f : 0.0;
+    }
+  }
+  __syncthreads();
+  // ---- symmetric orthonormalisation on 16 x 16 matrix tiles; wave w takes
+  // block column w
+  bool ql = false;
+  for (int it = 0; it < 4; ++it) {
+    double mx = 0.0;
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      tri_f64x4 e = {0.0, 0.0, 0.0, 0.0};
+#pragma unroll
+      for (int k = 0; k < 64; k += 4)
+        e = __builtin_amdgcn_mfma_f64_16x16x4f64(Z[(k + lk) * kAllLd + 16 * i + lr],
+                                                 Z[(k + lk) * kAllLd + 16 * wave + lr], e, 0, 0, 0);
+#pragma unroll
+      for (int v = 0; v < 4; ++v) {
+        const int p = 16 * i + lk + 4 * v, q = 16 * wave + lr;
+        const double x = p < n && q < n ? e[v] - (p == q ? 1.0 : 0.0) : 0.0;
+        U[p * kAllLd + q] = x;
+        mx = fmax(mx, fabs(x) <= 1e300 ? fabs(x) : 1e308);  // a NaN counts
+      }
+    }
+    for (int o = 32; o > 0; o >>= 1) mx = fmax(mx, __shfl_xor(mx, o, 64));
+    if (lane == 0) red[wave] = mx;
+    __syncthreads();
+    mx = fmax(fmax(red[0], red[1]), fmax(red[2], red[3]));
+    ql = it == 0 && mx > 1e-6;
+    if (ql || mx <= 1e-15) break;
+    tri_f64x4 z[4];
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      tri_f64x4 c = {0.0, 0.0, 0.0, 0.0};
+#pragma unroll
+      for (int k = 0; k < 64; k += 4)
+        c = __builtin_amdgcn_mfma_f64_16x16x4f64(Z[(16 * i + lr) * kAllLd + k + lk],
+                                                 U[(k + lk) * kAllLd + 16 * wave + lr], c, 0, 0, 0);
+#pragma unroll
+      for (int v = 0; v < 4; ++v) z[i][v] = fma(-0.5, c[v], Z[(16 * i + lk + 4 * v) * kAllLd + 16 * wave + lr]);
+    }
+    __syncthreads();
+#pragma unroll
+    for (int i = 0; i < 4; ++i)
+#pragma unroll
+      for (int v = 0; v < 4; ++v) Z[(16 * i + lk + 4 * v) * kAllLd + 16 * wave + lr] = z[i][v];
+    __syncthreads();
+  }
+  if (ql) {
+    __syncthreads();
+    if (wave == 0) tridiag_ql_wave(ad, bd, n, w, S, ldS, Z, part[0]);
+    return;
+  }
+  if (wave == 0 && lane < n) w[lane] = ldexp(lam, ex);
+  for (int k = wave; k < n; k += 4)
+    if (lane < n) S[k * ldS + lane] = Z[k * kAllLd + lane];
 }
 
 // ---------------------------------------------------------------------------
@@ -1967,7 +2147,7 @@ static int gd_correction(EigCtx& c, const float* V32, int J32, int keep, int m, 
   // within 0.1% of ||H||_est of the lowest (at least 2, at most `keep`): a
   // gapped spectrum needs a couple of FP64 matvecs here, a clustered one
   // keeps the whole cluster
-  hipLaunchKernelGGL(tridiag_all_kernel, dim3(1), dim3(64), 0, s, k.alpha, k.beta, J32, k.theta,
+  hipLaunchKernelGGL(tridiag_all_kernel, dim3(1), dim3(256), 0, s, k.alpha, k.beta, J32, k.theta,
                      k.S, kMaxBasis, kOne);
   TNX_LAUNCH_CHECK();
   std::vector<double> th(J32);
@@ -2305,7 +2485,7 @@ static int eigsh_run(EigCtx& c, const double* v0, double* vec, double* hvec,
         if (J >= mb) {
           // Thick restart keeping the `keep` lowest Ritz pairs in a basis
           // where the projected matrix stays tridiagonal.
-          hipLaunchKernelGGL(tridiag_all_kernel, dim3(1), dim3(64), 0, s, k.alpha, k.beta, J,
+          hipLaunchKernelGGL(tridiag_all_kernel, dim3(1), dim3(256), 0, s, k.alpha, k.beta, J,
                              k.theta, k.S, kMaxBasis, kOne);
           TNX_LAUNCH_CHECK();
           int* kp_dev = reinterpret_cast<int*>(k.st + 8);
@@ -2646,7 +2826,7 @@ int eigsh_heff1_b(const double* L, const double* W, const double* R, const doubl
       }
       if (Jl >= mb) {
         const int jl = Jl - 1;
-        hipLaunchKernelGGL(tridiag_all_kernel, dim3(1, cnt), dim3(64), 0, s, k.alpha, k.beta, Jl,
+        hipLaunchKernelGGL(tridiag_all_kernel, dim3(1, cnt), dim3(256), 0, s, k.alpha, k.beta, Jl,
                            k.theta, k.S, kMaxBasis, pm);
         TNX_LAUNCH_CHECK();
         hipLaunchKernelGGL(tr_restart_kernel, dim3(1, cnt), dim3(64), 0, s, k.theta, k.S, k.beta, jl,
@@ -2745,7 +2925,7 @@ int eigsh_heff1_b(const double* L, const double* W, const double* R, const doubl
       TNX_TRY(upload(idx, act));
     }
     if (J >= mb) {
-      hipLaunchKernelGGL(tridiag_all_kernel, dim3(1, cnt), dim3(64), 0, s, k.alpha, k.beta, J,
+      hipLaunchKernelGGL(tridiag_all_kernel, dim3(1, cnt), dim3(256), 0, s, k.alpha, k.beta, J,
                          k.theta, k.S, kMaxBasis, pm);
       TNX_LAUNCH_CHECK();
       hipLaunchKernelGGL(tr_restart_kernel, dim3(1, cnt), dim3(64), 0, s, k.theta, k.S, k.beta, j,
