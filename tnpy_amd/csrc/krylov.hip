@@ -44,10 +44,93 @@ int heff1_matvec_b(const void* L, const double* W, const void* R, const void* x,
                    hipStream_t s, int env_f32);
 size_t heff2_ws_bytes(int chil, int Dl, int Dm, int Dr, int d, int chir);
 
-__device__ __forceinline__ double wave_sum(double v) {
-#pragma unroll
-  for (int o = 32; o > 0; o >>= 1) v += __shfl_xor(v, o, 64);
-  return v;
+// Lane i's value of a wave-distributed double, as a wave-uniform scalar
+// (v_readlane: no LDS round trip). i must be wave-uniform.
+__device__ __forceinline__ double lane_val(double v, int i) {
+  const long long u = __double_as_longlong(v);
+  const unsigned lo = __builtin_amdgcn_readlane((int)(u & 0xffffffffll), i);
+  const unsigned hi = __builtin_amdgcn_readlane((int)(u >> 32), i);
+  return __longlong_as_double((long long)(((unsigned long long)hi << 32) | lo));
+}
+__device__ __forceinline__ int lane_int(int v, int i) { return __builtin_amdgcn_readlane(v, i); }
+
+// The value of the lane that a DPP control selects, `none` where there is
+// none. Reductions and scans over a wave go through these and lane reads: a
+// step costs a few cycles, where a shuffle waits for an LDS round trip.
+template <int CTRL>
+__device__ __forceinline__ double dpp(double x, double none = 0.0) {
+  const long long u = __double_as_longlong(x), w = __double_as_longlong(none);
+  const unsigned lo = __builtin_amdgcn_update_dpp((int)w, (int)u, CTRL, 0xf, 0xf, false);
+  const unsigned hi = __builtin_amdgcn_update_dpp((int)(w >> 32), (int)(u >> 32), CTRL, 0xf, 0xf, false);
+  return __longlong_as_double((long long)((unsigned long long)hi << 32 | lo));
+}
+
+// op over each 16 lanes, in all of them: neighbours, pairs, then the mirrored
+// halves; over the wave, the four groups by lane reads.
+template <typename OP>
+__device__ __forceinline__ double reduce16(double x, OP op) {
+  x = op(x, dpp<0xB1>(x));     // quad_perm 1 0 3 2
+  x = op(x, dpp<0x4E>(x));     // quad_perm 2 3 0 1
+  x = op(x, dpp<0x141>(x));    // row_half_mirror
+  return op(x, dpp<0x140>(x));  // row_mirror
+}
+
+template <typename OP>
+__device__ __forceinline__ double wave_reduce(double x, OP op) {
+  x = reduce16(x, op);
+  return op(op(lane_val(x, 0), lane_val(x, 16)), op(lane_val(x, 32), lane_val(x, 48)));
+}
+
+__device__ __forceinline__ double sum16(double x) {
+  return reduce16(x, [](double a, double b) { return a + b; });
+}
+__device__ __forceinline__ double wave_sum(double x) {
+  return wave_reduce(x, [](double a, double b) { return a + b; });
+}
+__device__ __forceinline__ double wave_min(double x) {
+  return wave_reduce(x, [](double a, double b) { return fmin(a, b); });
+}
+__device__ __forceinline__ double wave_max(double x) {
+  return wave_reduce(x, [](double a, double b) { return fmax(a, b); });
+}
+
+// Product of this lane's value and those of the lanes below it (above it).
+__device__ __forceinline__ double wave_prod_below(double f) {
+  f *= dpp<0x111>(f, 1.0);  // row_shr 1, 2, 4, 8
+  f *= dpp<0x112>(f, 1.0);
+  f *= dpp<0x114>(f, 1.0);
+  f *= dpp<0x118>(f, 1.0);
+  const double t0 = lane_val(f, 15), t1 = t0 * lane_val(f, 31), t2 = t1 * lane_val(f, 47);
+  const int row = (threadIdx.x & 63) >> 4;
+  return f * (row == 0 ? 1.0 : (row == 1 ? t0 : (row == 2 ? t1 : t2)));
+}
+__device__ __forceinline__ double wave_prod_above(double f) {
+  f *= dpp<0x101>(f, 1.0);  // row_shl 1, 2, 4, 8
+  f *= dpp<0x102>(f, 1.0);
+  f *= dpp<0x104>(f, 1.0);
+  f *= dpp<0x108>(f, 1.0);
+  const double t2 = lane_val(f, 48), t1 = t2 * lane_val(f, 32), t0 = t1 * lane_val(f, 16);
+  const int row = (threadIdx.x & 63) >> 4;
+  return f * (row == 3 ? 1.0 : (row == 2 ? t2 : (row == 1 ? t1 : t0)));
+}
+
+// x of the lower half of the wave beside y of the upper (HALF 32), or of the
+// even and odd rows of 16 (HALF 16), plus what each gets from the other:
+// lanes of the first kind return x + the partner's x, the others y + its y.
+template <int HALF>
+__device__ __forceinline__ double swap_add(double x, double y) {
+  const long long a = __double_as_longlong(x), b = __double_as_longlong(y);
+  double r[2];
+  if constexpr (HALF == 32) {
+    const auto lo = __builtin_amdgcn_permlane32_swap((unsigned)a, (unsigned)b, false, false);
+    const auto hi = __builtin_amdgcn_permlane32_swap((unsigned)(a >> 32), (unsigned)(b >> 32), false, false);
+    for (int q = 0; q < 2; ++q) r[q] = __longlong_as_double((long long)((unsigned long long)hi[q] << 32 | lo[q]));
+  } else {
+    const auto lo = __builtin_amdgcn_permlane16_swap((unsigned)a, (unsigned)b, false, false);
+    const auto hi = __builtin_amdgcn_permlane16_swap((unsigned)(a >> 32), (unsigned)(b >> 32), false, false);
+    for (int q = 0; q < 2; ++q) r[q] = __longlong_as_double((long long)((unsigned long long)hi[q] << 32 | lo[q]));
+  }
+  return r[0] + r[1];
 }
 
 // Problem map of a batched launch: launched problem i = blockIdx.y works on
@@ -385,20 +468,34 @@ __device__ __forceinline__ void sum_partials(const double* __restrict__ partials
 // v[0] is the total of row cgs_row_of<JW>(l) of the wave's rows.
 template <int JW>
 __device__ __forceinline__ double lane_totals(double (&v)[JW]) {
+  // halves of the wave, then rows of 16, by swaps; inside a row by DPP: lane
+  // ^ 8, then the mirrored 8 (^ 7), 4 (^ 3) and pairs, which between them
+  // also meet every lane once
   const int lane = threadIdx.x & 63;
+  static_assert(JW == 4 || JW == 8 || JW == 16, "two swapped levels, the rest inside a row");
+  auto other = [](double x, int o) {
+    return o == 8 ? dpp<0x128>(x) : (o == 4 ? dpp<0x141>(x) : (o == 2 ? dpp<0x1B>(x) : dpp<0xB1>(x)));
+  };
   int o = 32;
 #pragma unroll
   for (int c = JW / 2; c >= 1; c >>= 1) {
     const bool up = lane & o;
 #pragma unroll
     for (int k = 0; k < c; ++k) {
-      const double keep = up ? v[c + k] : v[k], send = up ? v[k] : v[c + k];
-      v[k] = keep + __shfl_xor(send, o, 64);
+      if (o == 32) {
+        v[k] = swap_add<32>(v[k], v[c + k]);
+      } else if (o == 16) {
+        v[k] = swap_add<16>(v[k], v[c + k]);
+      } else {
+        const double keep = up ? v[c + k] : v[k], send = up ? v[k] : v[c + k];
+        v[k] = keep + other(send, o);
+      }
     }
     o >>= 1;
   }
   double t = v[0];
-  for (; o > 0; o >>= 1) t += __shfl_xor(t, o, 64);
+#pragma unroll
+  for (; o > 0; o >>= 1) t += other(t, o);
   return t;
 }
 
@@ -655,16 +752,6 @@ __global__ void copy_map_kernel(const double* __restrict__ in, double* __restric
 // ---------------------------------------------------------------------------
 constexpr int kTriMax = 256;
 
-// Lane i's value of a wave-distributed double, as a wave-uniform scalar
-// (v_readlane: no LDS round trip). i must be wave-uniform.
-__device__ __forceinline__ double lane_val(double v, int i) {
-  const long long u = __double_as_longlong(v);
-  const unsigned lo = __builtin_amdgcn_readlane((int)(u & 0xffffffffll), i);
-  const unsigned hi = __builtin_amdgcn_readlane((int)(u >> 32), i);
-  return __longlong_as_double((long long)(((unsigned long long)hi << 32) | lo));
-}
-__device__ __forceinline__ int lane_int(int v, int i) { return __builtin_amdgcn_readlane(v, i); }
-
 // Orders one wave's LDS writes before its later reads of other lanes'
 // values (LDS serves a wave's instructions in order; this keeps the compiler
 // from moving them).
@@ -805,11 +892,9 @@ __device__ __forceinline__ void tridiag_lowest_wave(TriLds& t, const double* __r
   }
   if (lane < 16) t.row[64 * NC + lane] = make_double2(0.0, 0.0);
   wave_lds_fence();
-  for (int o = 32; o > 0; o >>= 1) {
-    lo = fmin(lo, __shfl_xor(lo, o, 64));
-    hi = fmin(hi, __shfl_xor(hi, o, 64));
-    tnorm = fmax(tnorm, __shfl_xor(tnorm, o, 64));
-  }
+  lo = wave_min(lo);
+  hi = wave_min(hi);
+  tnorm = wave_max(tnorm);
   // far from 1 the products of rows would leave the range: by a power of two
   int ex = __builtin_amdgcn_frexp_exp(tnorm);
   if (ex < -64 || ex > 64) {
@@ -923,7 +1008,7 @@ __device__ __forceinline__ void tridiag_lowest_wave(TriLds& t, const double* __r
     }
     gmin = fmin(gmin, gam[c]);
   }
-  for (int o = 32; o > 0; o >>= 1) gmin = fmin(gmin, __shfl_xor(gmin, o, 64));
+  gmin = wave_min(gmin);
   int r = -1;
 #pragma unroll
   for (int c = 0; c < NC; ++c) {
@@ -935,12 +1020,8 @@ __device__ __forceinline__ void tridiag_lowest_wave(TriLds& t, const double* __r
 #pragma unroll
   for (int c = 0; c < NC; ++c) {
     const int k = 64 * c + lane;
-    double f = k > r && k < n ? dn[c] : 1.0;
-    for (int o = 1; o < 64; o <<= 1) {
-      const double v = __shfl_up(f, o, 64);
-      if (lane >= o) f *= v;
-    }
-    z[c] = f * carry;
+    const double f = k > r && k < n ? dn[c] : 1.0;
+    z[c] = wave_prod_below(f) * carry;
     if (NC > 1) carry = lane_val(z[c], 63);
   }
   // above r: running products upwards
@@ -948,12 +1029,7 @@ __device__ __forceinline__ void tridiag_lowest_wave(TriLds& t, const double* __r
 #pragma unroll
   for (int c = NC - 1; c >= 0; --c) {
     const int k = 64 * c + lane;
-    double f = k < r ? up[c] : 1.0;
-    for (int o = 1; o < 64; o <<= 1) {
-      const double v = __shfl_down(f, o, 64);
-      if (lane + o < 64) f *= v;
-    }
-    f *= carry;
+    const double f = wave_prod_above(k < r ? up[c] : 1.0) * carry;
     if (NC > 1) carry = lane_val(f, 0);
     z[c] = k < n ? z[c] * f : 0.0;
   }
@@ -963,10 +1039,8 @@ __device__ __forceinline__ void tridiag_lowest_wave(TriLds& t, const double* __r
     nn += z[c] * z[c];
     mx = fmax(mx, fabs(z[c]));
   }
-  for (int o = 32; o > 0; o >>= 1) {
-    nn += __shfl_xor(nn, o, 64);
-    mx = fmax(mx, __shfl_xor(mx, o, 64));
-  }
+  nn = wave_sum(nn);
+  mx = wave_max(mx);
   // unit length; sign: largest |component| positive, the first such index on
   // ties
   double sg = 1.0 / sqrt(nn), zl = 0.0;
@@ -1145,29 +1219,6 @@ static int finish_step(VT* V, int64_t N, int J, const double* w, const double* p
 // Dense symmetric tridiagonalisation (one workgroup) and back-transform.
 // Householder reflectors H_k = I - tau_k v_k v_k^T act on indices k+1..n-1.
 // ---------------------------------------------------------------------------
-// Lanes a DPP control selects, added (both halves of a double).
-template <int CTRL>
-__device__ __forceinline__ double dpp_add(double x) {
-  const long long u = __double_as_longlong(x);
-  const unsigned lo = __builtin_amdgcn_update_dpp(0, (int)u, CTRL, 0xf, 0xf, true);
-  const unsigned hi = __builtin_amdgcn_update_dpp(0, (int)(u >> 32), CTRL, 0xf, 0xf, true);
-  return x + __longlong_as_double((long long)((unsigned long long)hi << 32 | lo));
-}
-
-// Sum over each group of 16 lanes, in all of them: neighbours, pairs, then
-// the mirrored halves.
-__device__ __forceinline__ double sum16(double x) {
-  x = dpp_add<0xB1>(x);   // quad_perm 1 0 3 2
-  x = dpp_add<0x4E>(x);   // quad_perm 2 3 0 1
-  x = dpp_add<0x141>(x);  // row_half_mirror
-  return dpp_add<0x140>(x);  // row_mirror
-}
-
-__device__ __forceinline__ double sum64(double x) {
-  x = sum16(x);
-  return (lane_val(x, 0) + lane_val(x, 16)) + (lane_val(x, 32) + lane_val(x, 48));
-}
-
 // Tridiagonalisation with the matrix in registers: 16 lanes hold R rows, C
 // elements of each (in pairs of columns), so a step is two barriers: the
 // product p = tau A v with v from LDS (sums inside the 16 lanes), and the
@@ -1267,7 +1318,7 @@ __global__ __launch_bounds__(16 * NG) void sytrd_reg_kernel(const double* __rest
       part[g] = pv;
     }
     __syncthreads();
-    const double K = 0.5 * tk * sum64(lane < NG ? part[lane] : 0.0);
+    const double K = 0.5 * tk * wave_sum(lane < NG ? part[lane] : 0.0);
     double wj[C];
 #pragma unroll
     for (int c = 0; c < C; ++c) wj[c] = fma(-K, vj[c], p[col(c)]);
@@ -1409,7 +1460,7 @@ __global__ __launch_bounds__(64) void ormtr_kernel(const double* __restrict__ Vs
       double d = 0.0;
 #pragma unroll
       for (int q = 0; q < Q; ++q) d = fma(w[u][q], xs[q], d);
-      d = -f[u] * sum64(d);
+      d = -f[u] * wave_sum(d);
 #pragma unroll
       for (int q = 0; q < Q; ++q) xs[q] = fma(d, w[u][q], xs[q]);
     }
@@ -1615,7 +1666,7 @@ __global__ __launch_bounds__(256) void tridiag_all_kernel(const double* __restri
   double a = lane < n ? ad[lane] : 0.0, b = lane < n - 1 ? bd[lane] : 0.0;
   double bl = lane > 0 && lane < n ? bd[lane - 1] : 0.0;
   double r0 = fabs(b) + fabs(bl), tn = lane < n ? fabs(a) + r0 : 0.0;
-  for (int o = 32; o > 0; o >>= 1) tn = fmax(tn, __shfl_xor(tn, o, 64));
+  tn = wave_max(tn);
   int ex = __builtin_amdgcn_frexp_exp(tn);
   if (ex >= -64 && ex <= 64) ex = 0;
   a = ldexp(a, -ex);
@@ -1625,10 +1676,8 @@ __global__ __launch_bounds__(256) void tridiag_all_kernel(const double* __restri
   tn = ldexp(tn, -ex);
   const double eps = 2.220446049250313e-16;
   double lo = lane < n ? a - r0 : 1e308, hi = lane < n ? a + r0 : -1e308;
-  for (int o = 32; o > 0; o >>= 1) {
-    lo = fmin(lo, __shfl_xor(lo, o, 64));
-    hi = fmax(hi, __shfl_xor(hi, o, 64));
-  }
+  lo = wave_min(lo);
+  hi = wave_max(hi);
   lo -= 4.0 * eps * tn + 1e-300;
   hi += 4.0 * eps * tn + 1e-300;
   if (wave == 0) {
@@ -1743,7 +1792,7 @@ __global__ __launch_bounds__(256) void tridiag_all_kernel(const double* __restri
         mx = fmax(mx, fabs(x) <= 1e300 ? fabs(x) : 1e308);  // a NaN counts
       }
     }
-    for (int o = 32; o > 0; o >>= 1) mx = fmax(mx, __shfl_xor(mx, o, 64));
+    mx = wave_max(mx);
     if (lane == 0) red[wave] = mx;
     __syncthreads();
     mx = fmax(fmax(red[0], red[1]), fmax(red[2], red[3]));
@@ -1915,7 +1964,7 @@ __global__ __launch_bounds__(64) void tr_restart_kernel(const double* __restrict
   const double cl = (l < k) ? bj * S[j * kMaxBasis + l] : 0.0;
   const double th = (l < k) ? theta[l] : 0.0;
   double tmax = fabs(th);
-  for (int o = 32; o > 0; o >>= 1) tmax = fmax(tmax, __shfl_xor(tmax, o, 64));
+  tmax = wave_max(tmax);
   const double cn = sqrt(wave_sum(cl * cl));
   double qi = (cn > 0.0) ? cl / cn : (l == 0 ? 1.0 : 0.0);
   if (l < kMaxBasis) q[0][l] = (l < k) ? qi : 0.0;
