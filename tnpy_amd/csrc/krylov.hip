@@ -84,7 +84,7 @@ __device__ __forceinline__ double wave_reduce(double x, OP op) {
 __device__ __forceinline__ double sum16(double x) {
   return reduce16(x, [](double a, double b) { return a + b; });
 }
-__device__ __forceinline__ double wave_sum(double x) {
+__device__ __forceinline__ double sum64(double x) {
   return wave_reduce(x, [](double a, double b) { return a + b; });
 }
 __device__ __forceinline__ double wave_min(double x) {
@@ -92,26 +92,6 @@ __device__ __forceinline__ double wave_min(double x) {
 }
 __device__ __forceinline__ double wave_max(double x) {
   return wave_reduce(x, [](double a, double b) { return fmax(a, b); });
-}
-
-// Product of this lane's value and those of the lanes below it (above it).
-__device__ __forceinline__ double wave_prod_below(double f) {
-  f *= dpp<0x111>(f, 1.0);  // row_shr 1, 2, 4, 8
-  f *= dpp<0x112>(f, 1.0);
-  f *= dpp<0x114>(f, 1.0);
-  f *= dpp<0x118>(f, 1.0);
-  const double t0 = lane_val(f, 15), t1 = t0 * lane_val(f, 31), t2 = t1 * lane_val(f, 47);
-  const int row = (threadIdx.x & 63) >> 4;
-  return f * (row == 0 ? 1.0 : (row == 1 ? t0 : (row == 2 ? t1 : t2)));
-}
-__device__ __forceinline__ double wave_prod_above(double f) {
-  f *= dpp<0x101>(f, 1.0);  // row_shl 1, 2, 4, 8
-  f *= dpp<0x102>(f, 1.0);
-  f *= dpp<0x104>(f, 1.0);
-  f *= dpp<0x108>(f, 1.0);
-  const double t2 = lane_val(f, 48), t1 = t2 * lane_val(f, 32), t0 = t1 * lane_val(f, 16);
-  const int row = (threadIdx.x & 63) >> 4;
-  return f * (row == 3 ? 1.0 : (row == 2 ? t2 : (row == 1 ? t1 : t0)));
 }
 
 // x of the lower half of the wave beside y of the upper (HALF 32), or of the
@@ -131,6 +111,17 @@ __device__ __forceinline__ double swap_add(double x, double y) {
     for (int q = 0; q < 2; ++q) r[q] = __longlong_as_double((long long)((unsigned long long)hi[q] << 32 | lo[q]));
   }
   return r[0] + r[1];
+}
+
+// Sum over the wave in all lanes, as the tree of lane ^ 32, ^ 16, ... ^ 1 (once
+// the sums repeat every 8 or 4 lanes, a rotation reaches the same partner).
+__device__ __forceinline__ double wave_sum(double x) {
+  x = swap_add<32>(x, x);
+  x = swap_add<16>(x, x);
+  x += dpp<0x128>(x);  // row_ror 8, 4
+  x += dpp<0x124>(x);
+  x += dpp<0x4E>(x);  // quad_perm 2 3 0 1, 1 0 3 2
+  return x + dpp<0xB1>(x);
 }
 
 // Problem map of a batched launch: launched problem i = blockIdx.y works on
@@ -468,13 +459,16 @@ __device__ __forceinline__ void sum_partials(const double* __restrict__ partials
 // v[0] is the total of row cgs_row_of<JW>(l) of the wave's rows.
 template <int JW>
 __device__ __forceinline__ double lane_totals(double (&v)[JW]) {
-  // halves of the wave, then rows of 16, by swaps; inside a row by DPP: lane
-  // ^ 8, then the mirrored 8 (^ 7), 4 (^ 3) and pairs, which between them
-  // also meet every lane once
+  // halves of the wave, then rows of 16, by swaps; inside a row by DPP
   const int lane = threadIdx.x & 63;
   static_assert(JW == 4 || JW == 8 || JW == 16, "two swapped levels, the rest inside a row");
-  auto other = [](double x, int o) {
-    return o == 8 ? dpp<0x128>(x) : (o == 4 ? dpp<0x141>(x) : (o == 2 ? dpp<0x1B>(x) : dpp<0xB1>(x)));
+  auto other = [&](double x, int o) {  // of lane ^ o
+    if (o == 8) return dpp<0x128>(x);
+    if (o == 4) {
+      const double before = dpp<0x124>(x), behind = dpp<0x12C>(x);
+      return lane & 4 ? before : behind;
+    }
+    return o == 2 ? dpp<0x4E>(x) : dpp<0xB1>(x);
   };
   int o = 32;
 #pragma unroll
@@ -1020,8 +1014,12 @@ __device__ __forceinline__ void tridiag_lowest_wave(TriLds& t, const double* __r
 #pragma unroll
   for (int c = 0; c < NC; ++c) {
     const int k = 64 * c + lane;
-    const double f = k > r && k < n ? dn[c] : 1.0;
-    z[c] = wave_prod_below(f) * carry;
+    double f = k > r && k < n ? dn[c] : 1.0;
+    for (int o = 1; o < 64; o <<= 1) {
+      const double v = __shfl_up(f, o, 64);
+      if (lane >= o) f *= v;
+    }
+    z[c] = f * carry;
     if (NC > 1) carry = lane_val(z[c], 63);
   }
   // above r: running products upwards
@@ -1029,7 +1027,12 @@ __device__ __forceinline__ void tridiag_lowest_wave(TriLds& t, const double* __r
 #pragma unroll
   for (int c = NC - 1; c >= 0; --c) {
     const int k = 64 * c + lane;
-    const double f = wave_prod_above(k < r ? up[c] : 1.0) * carry;
+    double f = k < r ? up[c] : 1.0;
+    for (int o = 1; o < 64; o <<= 1) {
+      const double v = __shfl_down(f, o, 64);
+      if (lane + o < 64) f *= v;
+    }
+    f *= carry;
     if (NC > 1) carry = lane_val(f, 0);
     z[c] = k < n ? z[c] * f : 0.0;
   }
@@ -1318,7 +1321,7 @@ __global__ __launch_bounds__(16 * NG) void sytrd_reg_kernel(const double* __rest
       part[g] = pv;
     }
     __syncthreads();
-    const double K = 0.5 * tk * wave_sum(lane < NG ? part[lane] : 0.0);
+    const double K = 0.5 * tk * sum64(lane < NG ? part[lane] : 0.0);
     double wj[C];
 #pragma unroll
     for (int c = 0; c < C; ++c) wj[c] = fma(-K, vj[c], p[col(c)]);
@@ -1460,7 +1463,7 @@ __global__ __launch_bounds__(64) void ormtr_kernel(const double* __restrict__ Vs
       double d = 0.0;
 #pragma unroll
       for (int q = 0; q < Q; ++q) d = fma(w[u][q], xs[q], d);
-      d = -f[u] * wave_sum(d);
+      d = -f[u] * sum64(d);
 #pragma unroll
       for (int q = 0; q < Q; ++q) xs[q] = fma(d, w[u][q], xs[q]);
     }
