@@ -61,15 +61,13 @@ __device__ __forceinline__ double jac_dpp(double x) {
   return __longlong_as_double((long long)((unsigned long long)hi << 32 | lo));
 }
 
-// One sweep of two-sided cyclic Jacobi on each pair's Gram matrix G (kJp x
-// kJp, row-major); Z accumulates the rotations (G_final = Z^T G Z). Rotation l
+// One sweep of two-sided cyclic Jacobi on a pair's Gram matrix G (kJp x kJp);
+// Z accumulates the rotations (G_final = Z^T G Z). Rotation l
 // of a round takes places e_l and o_l (rows l and kJw + l at the start), and
 // after it the rows move on: in a full sweep (kJp - 1 rounds, every pair
 // once) by the round-robin tournament, e_0 fixed; with CROSS (kJw rounds,
 // the pairs of a row of one block with one of the other) o_l takes o_(l+1).
-// Both are back in place after the last round. Also the pair's off-diagonal
-// measure, max-reduced into *off_bits (a non-negative double read as an
-// unsigned integer, so integer max = double max).
+// Both are back in place after the last round.
 //
 // Everything stays in registers. Threads 0..255, in 16 x 16, hold 4 x 4
 // entries of G each (two rotations' rows and columns): the 16 with a diagonal
@@ -79,62 +77,67 @@ __device__ __forceinline__ double jac_dpp(double x) {
 // a round: 55 us for the 63 rounds of a full sweep. With G and Z in LDS and the
 // rotations addressed by index 98 us; with correctly rounded angles, both of a
 // block's by its own lane, 90.
-template <bool CROSS>
-__global__ __launch_bounds__(512) void jacobi_pair_kernel(const double* __restrict__ Gall,
-                                                         double* __restrict__ Zall,
-                                                         const double* __restrict__ floor2,
-                                                         unsigned long long* __restrict__ off_bits) {
-  __shared__ __attribute__((aligned(32))) jac_f64x4 xe[256], xo[256];  // rows on their way
-  __shared__ __attribute__((aligned(16))) jac_f64x2 cs[2][kJw];
-  __shared__ double dg[kJp], red[4];
-  const int tid = threadIdx.x;
-  const bool inz = tid >= 256;
-  const int tx = tid & 15, ty = (tid >> 4) & 15;      // of G
-  const int zr = (tid & 255) >> 2, zq = tid & 3;      // row and quarter of Z
-  const double* Gp = Gall + (size_t)blockIdx.x * kJp * kJp;
-  auto place = [](int pair, int h) { return pair + kJw * h; };
-  // x[r][c]: row pair 2 ty + r / 2, column pair 2 tx + c / 2 (h = r % 2, c % 2)
-  // of G; for Z x[i / 4][i % 4] is pair 8 zq + i / 2, h = i % 2
-  double x[4][4];
+struct JacLds {
+  jac_f64x4 xe[256], xo[256];  // rows on their way
+  jac_f64x2 cs[2][kJw];
+  double dg[kJp], red[4];
+};
+
+__device__ __forceinline__ int jac_place(int pair, int h) { return pair + kJw * h; }
+
+// The entries of this thread: x[r][c] of row pair 2 ty + r / 2, column pair 2
+// tx + c / 2 (h = r % 2, c % 2) of G = (g + g^T) / 2; for Z (threads from 256)
+// x[i / 4][i % 4] of pair 8 zq + i / 2, h = i % 2, the identity.
+template <typename F>
+__device__ __forceinline__ void jac_load(double (&x)[4][4], F g) {
+  const int tid = threadIdx.x, tx = tid & 15, ty = (tid >> 4) & 15, zr = (tid & 255) >> 2, zq = tid & 3;
 #pragma unroll
   for (int r = 0; r < 4; ++r)
 #pragma unroll
     for (int c = 0; c < 4; ++c) {
-      if (inz) {
+      if (tid >= 256) {
         const int i = 4 * r + c;
-        x[r][c] = place(8 * zq + (i >> 1), i & 1) == zr ? 1.0 : 0.0;
+        x[r][c] = jac_place(8 * zq + (i >> 1), i & 1) == zr ? 1.0 : 0.0;
       } else {
-        // symmetrise (the GEMM's two halves round independently)
-        const int i = place(2 * ty + (r >> 1), r & 1), j = place(2 * tx + (c >> 1), c & 1);
-        x[r][c] = 0.5 * (Gp[i * kJp + j] + Gp[j * kJp + i]);
+        const int i = jac_place(2 * ty + (r >> 1), r & 1), j = jac_place(2 * tx + (c >> 1), c & 1);
+        x[r][c] = 0.5 * (g(i, j) + g(j, i));
       }
     }
-  // ---- off-diagonal measure of the incoming pair: |G_ij| over the larger of
-  // sqrt(G_ii G_jj) and the floor
-  if (!inz && tx == ty) {
+}
+
+// Off-diagonal measure of G: the largest |G_ij| over the larger of sqrt(G_ii
+// G_jj) and the floor, in all threads.
+__device__ __forceinline__ double jac_off(const double (&x)[4][4], double floor2, JacLds& s) {
+  const int tid = threadIdx.x, tx = tid & 15, ty = (tid >> 4) & 15;
+  if (tid < 256 && tx == ty) {
 #pragma unroll
-    for (int r = 0; r < 4; ++r) dg[place(2 * ty + (r >> 1), r & 1)] = rsqrt_nr(fmax(x[r][r], 1e-300));
+    for (int r = 0; r < 4; ++r) s.dg[jac_place(2 * ty + (r >> 1), r & 1)] = rsqrt_nr(fmax(x[r][r], 1e-300));
   }
   __syncthreads();
-  if (!inz) {
-    const double ifl = 1.0 / floor2[0];
+  if (tid < 256) {
+    const double ifl = 1.0 / floor2;
     double mx = 0.0;
 #pragma unroll
     for (int r = 0; r < 4; ++r)
 #pragma unroll
       for (int c = 0; c < 4; ++c) {
-        const int i = place(2 * ty + (r >> 1), r & 1), j = place(2 * tx + (c >> 1), c & 1);
-        const double o = fabs(x[r][c]) * fmin(dg[i] * dg[j], ifl);
+        const int i = jac_place(2 * ty + (r >> 1), r & 1), j = jac_place(2 * tx + (c >> 1), c & 1);
+        const double o = fabs(x[r][c]) * fmin(s.dg[i] * s.dg[j], ifl);
         mx = i != j ? fmax(mx, o) : mx;
       }
 #pragma unroll
     for (int o = 32; o > 0; o >>= 1) mx = fmax(mx, __shfl_xor(mx, o, 64));
-    if ((tid & 63) == 0) red[tid >> 6] = mx;
+    if ((tid & 63) == 0) s.red[tid >> 6] = mx;
   }
   __syncthreads();
-  if (tid == 0)
-    atomicMax(off_bits,
-              (unsigned long long)__double_as_longlong(fmax(fmax(red[0], red[1]), fmax(red[2], red[3]))));
+  return fmax(fmax(s.red[0], s.red[1]), fmax(s.red[2], s.red[3]));
+}
+
+template <bool CROSS>
+__device__ __forceinline__ void jac_sweep(double (&x)[4][4], JacLds& s) {
+  const int tid = threadIdx.x;
+  const bool inz = tid >= 256;
+  const int tx = tid & 15, ty = (tid >> 4) & 15, zq = tid & 3;
   constexpr int rounds = CROSS ? kJw : kJp - 1;
   if (inz) {
     double* z = &x[0][0];
@@ -143,7 +146,7 @@ __global__ __launch_bounds__(512) void jacobi_pair_kernel(const double* __restri
       // Z <- Z J, then the columns move on
 #pragma unroll
       for (int l = 0; l < 8; ++l) {
-        const jac_f64x2 v = cs[r & 1][8 * zq + l];
+        const jac_f64x2 v = s.cs[r & 1][8 * zq + l];
         const double e = z[2 * l], o = z[2 * l + 1];
         z[2 * l] = v[0] * e - v[1] * o;
         z[2 * l + 1] = v[1] * e + v[0] * o;
@@ -162,9 +165,6 @@ __global__ __launch_bounds__(512) void jacobi_pair_kernel(const double* __restri
       }
       __syncthreads();
     }
-    double* Zp = Zall + (size_t)blockIdx.x * kJp * kJp;
-#pragma unroll
-    for (int i = 0; i < 16; ++i) Zp[zr * kJp + place(8 * zq + (i >> 1), i & 1)] = z[i];
     return;
   }
   // the second rotation of a diagonal block is worked out by the next lane
@@ -183,10 +183,10 @@ __global__ __launch_bounds__(512) void jacobi_pair_kernel(const double* __restri
       const double v = fma(u, q1, fabs(zeta)), p0 = __builtin_amdgcn_rcp(v), p1 = fma(p0, fma(-v, p0, 1.0), p0);
       const double t = zeta >= 0.0 ? p1 : -p1, c = rsqrt_nr(fma(t, t, 1.0));
       const bool on = b != 0.0 && fabs(zeta) < 1e100;
-      cs[r & 1][2 * ty + own] = jac_f64x2{on ? c : 1.0, on ? c * t : 0.0};
+      s.cs[r & 1][2 * ty + own] = jac_f64x2{on ? c : 1.0, on ? c * t : 0.0};
     }
     __syncthreads();
-    const jac_f64x2* w = cs[r & 1];
+    const jac_f64x2* w = s.cs[r & 1];
     const jac_f64x2 kr[2] = {w[2 * ty], w[2 * ty + 1]}, lc[2] = {w[2 * tx], w[2 * tx + 1]};
 #pragma unroll
     for (int k = 0; k < 2; ++k)
@@ -218,12 +218,12 @@ __global__ __launch_bounds__(512) void jacobi_pair_kernel(const double* __restri
       }
     }
     // rows move between rows of threads
-    xo[tid] = jac_f64x4{x[1][0], x[1][1], x[1][2], x[1][3]};
-    if (!CROSS) xe[tid] = jac_f64x4{x[2][0], x[2][1], x[2][2], x[2][3]};
+    s.xo[tid] = jac_f64x4{x[1][0], x[1][1], x[1][2], x[1][3]};
+    if (!CROSS) s.xe[tid] = jac_f64x4{x[2][0], x[2][1], x[2][2], x[2][3]};
     __syncthreads();
-    const jac_f64x4 oi = xo[(tid + 16) & 255];
+    const jac_f64x4 oi = s.xo[(tid + 16) & 255];
     jac_f64x4 ei = {0.0, 0.0, 0.0, 0.0};
-    if (!CROSS) ei = xe[(tid + 240) & 255];
+    if (!CROSS) ei = s.xe[(tid + 240) & 255];
 #pragma unroll
     for (int j = 0; j < 4; ++j) {
       const double e0 = x[0][j], o0 = x[1][j], e1 = x[2][j], o1 = x[3][j];
@@ -235,6 +235,96 @@ __global__ __launch_bounds__(512) void jacobi_pair_kernel(const double* __restri
       }
     }
   }
+}
+
+// Z's entries of this thread to Z (row stride ld).
+__device__ __forceinline__ void jac_store_z(const double (&x)[4][4], double* Z, int ld) {
+  const int tid = threadIdx.x, zr = (tid & 255) >> 2, zq = tid & 3;
+  if (tid < 256) return;
+#pragma unroll
+  for (int i = 0; i < 16; ++i) Z[zr * ld + jac_place(8 * zq + (i >> 1), i & 1)] = x[i >> 2][i & 3];
+}
+
+// A sweep of every pair of a round, and the largest off-diagonal measure into
+// *off_bits (a non-negative double read as an unsigned integer, so integer
+// max = double max).
+template <bool CROSS>
+__global__ __launch_bounds__(512) void jacobi_pair_kernel(const double* __restrict__ Gall,
+                                                         double* __restrict__ Zall,
+                                                         const double* __restrict__ floor2,
+                                                         unsigned long long* __restrict__ off_bits) {
+  __shared__ __attribute__((aligned(32))) JacLds s;
+  const double* Gp = Gall + (size_t)blockIdx.x * kJp * kJp;
+  double x[4][4];
+  jac_load(x, [&](int i, int j) { return Gp[i * kJp + j]; });
+  const double off = jac_off(x, floor2[0], s);
+  if (threadIdx.x == 0) atomicMax(off_bits, (unsigned long long)__double_as_longlong(off));
+  jac_sweep<CROSS>(x, s);
+  jac_store_z(x, Zall + (size_t)blockIdx.x * kJp * kJp, kJp);
+}
+
+// One block pair alone (p, q <= kJp): every sweep in one launch, the rows in
+// LDS, their Gram matrix and rotation on 16 x 16 matrix tiles (two per wave).
+// With five launches and a host read per sweep a 64 x 64 core took 95 us a
+// sweep of which the rotations are 55.
+__global__ __launch_bounds__(512) void jacobi_one_kernel(const double* __restrict__ X0, int p, int q,
+                                                        double* __restrict__ Xout, int* __restrict__ sweeps) {
+  constexpr int ld = kJp + 1;
+  __shared__ __attribute__((aligned(32))) JacLds s;
+  __shared__ double X[kJp * ld], G[kJp * ld];
+  __shared__ double red[8];
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, lr = lane & 15, lk = lane >> 4;
+  double nn = 0.0;
+  for (int e = tid; e < kJp * kJp; e += 512) {
+    const int i = e >> 6, j = e & (kJp - 1);
+    const double v = i < p && j < q ? X0[(int64_t)i * q + j] : 0.0;
+    X[i * ld + j] = v;
+    nn = fma(v, v, nn);
+  }
+#pragma unroll
+  for (int o = 32; o > 0; o >>= 1) nn += __shfl_xor(nn, o, 64);
+  if (lane == 0) red[wave] = nn;
+  __syncthreads();
+  const double floor2 = kJacFloor * (((red[0] + red[1]) + (red[2] + red[3])) + ((red[4] + red[5]) + (red[6] + red[7])));
+  const int ti = 16 * (wave >> 1), tj = 32 * (wave & 1);  // two tiles side by side
+  int n = 0;
+  while (n < kJacMaxSweeps) {
+    ++n;
+    jac_f64x4 c[2] = {{0.0, 0.0, 0.0, 0.0}, {0.0, 0.0, 0.0, 0.0}};
+    for (int k = lk; k < kJp; k += 4)
+#pragma unroll
+      for (int u = 0; u < 2; ++u)
+        c[u] = __builtin_amdgcn_mfma_f64_16x16x4f64(X[(ti + lr) * ld + k], X[(tj + 16 * u + lr) * ld + k], c[u], 0, 0, 0);
+#pragma unroll
+    for (int u = 0; u < 2; ++u)
+#pragma unroll
+      for (int v = 0; v < 4; ++v) G[(ti + lk + 4 * v) * ld + tj + 16 * u + lr] = c[u][v];
+    __syncthreads();
+    double x[4][4];
+    jac_load(x, [&](int i, int j) { return G[i * ld + j]; });
+    const double off = jac_off(x, floor2, s);  // its barriers end the reads of G
+    jac_sweep<false>(x, s);
+    jac_store_z(x, G, ld);
+    __syncthreads();
+#pragma unroll
+    for (int u = 0; u < 2; ++u) c[u] = jac_f64x4{0.0, 0.0, 0.0, 0.0};
+    for (int k = lk; k < kJp; k += 4)
+#pragma unroll
+      for (int u = 0; u < 2; ++u)
+        c[u] = __builtin_amdgcn_mfma_f64_16x16x4f64(G[k * ld + ti + lr], X[k * ld + tj + 16 * u + lr], c[u], 0, 0, 0);
+    __syncthreads();
+#pragma unroll
+    for (int u = 0; u < 2; ++u)
+#pragma unroll
+      for (int v = 0; v < 4; ++v) X[(ti + lk + 4 * v) * ld + tj + 16 * u + lr] = c[u][v];
+    __syncthreads();
+    if (!(off > kJacTol)) break;
+  }
+  for (int e = tid; e < kJp * q; e += 512) {
+    const int i = e / q, j = e - i * q;
+    Xout[e] = X[i * ld + j];
+  }
+  if (tid == 0) *sweeps = n;
 }
 
 __global__ void jacobi_permute_kernel(const double* __restrict__ src, double* __restrict__ dst,
@@ -345,6 +435,15 @@ static int jacobi_rows(const double* X0, int p, int q, void* ws, double** Xout, 
   int* perm = (int*)w; w += al((size_t)B * 4);
   unsigned long long* off_bits = (unsigned long long*)w;
   double* floor2 = (double*)(w + 8);
+  if (B == 2 && q <= kJp) {
+    int* n = reinterpret_cast<int*>(off_bits);
+    hipLaunchKernelGGL(jacobi_one_kernel, dim3(1), dim3(512), 0, s, X0, p, q, X, n);
+    TNX_LAUNCH_CHECK();
+    TNX_HIP(hipMemcpyAsync(sweeps_out, n, sizeof(int), hipMemcpyDeviceToHost, s));
+    TNX_HIP(hipStreamSynchronize(s));
+    *Xout = X;
+    return TNX_OK;
+  }
   // round-robin position map (block 0 fixed, the others rotate)
   {
     const int h = B / 2;
