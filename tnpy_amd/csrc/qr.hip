@@ -500,8 +500,9 @@ __global__ __launch_bounds__(256) void qr_small_kernel(double* __restrict__ A, i
 // and takes the Householder steps. R's block column w stays in
 // wave w's registers. Bound by the chain of pivots (16 n per pass) and one
 // CU's matrix rate. The gauge move of a 60 x 2 x 60 site, with R times the
-// neighbour: 162 us with two panels of the many-workgroup path, 79 us so; a
-// batch of 64 x 2 x 64 sites took 683 us in the Householder kernel above.
+// neighbour: 162 us with two panels of a many-workgroup path, 54 us so (49 in
+// this kernel); 16 sites of 64 x 2 x 64 took 683 us in the Householder kernel
+// above, 66 here.
 constexpr int kQcLdsBig = 20200, kQcLdsLittle = 4864;  // 158 and 38 KiB
 
 template <int CAP, int NT, int NB>
