@@ -17,7 +17,7 @@ precision. The order:
    ``roofline`` object), and the QR gauge move.
 2. Warm state, untimed: one-site DMRG at ``--warm-chi`` from a seeded
    random MPS until the energy changes by less than tol (a bond-dimension
-   ramp), then the bonds are widened to chi (zero padding, Householder LQ
+   ramp), then the bonds are widened to chi (zero padding, LQ
    sweep: every chi=1024 tensor is a full orthonormal basis) and ``--warmup``
    FP64 sweeps run at chi. The reference's own sweep clock is the mean of
    the fastest sweeps of a run (``tnpy/finite_dmrg.py:252-256``): the

@@ -317,8 +317,9 @@ int tnx_eigsh_gen_heff1(const double* L, const double* W, const double* R, const
 int tnx_mpo_apply_site(const double* W, const double* A, int Dl, int Dr, int d, int l, int r,
                        double* out, tnx_stream_t stream);
 
-/* Householder QR of a row-major m x n matrix, m >= n: A <- Q (m x n,
- * orthonormal columns), R (n x n, upper triangular, row-major).
+/* QR of a row-major m x n matrix, m >= n: A <- Q (m x n, orthonormal
+ * columns), R (n x n, upper triangular with a non-negative diagonal,
+ * row-major).
  * Building block of the gauge moves (numpy.linalg.qr / LAPACK dgeqrf+dorgqr,
  * tnpy/linalg.py:26-39). */
 size_t tnx_qr_workspace_bytes(int m, int n);

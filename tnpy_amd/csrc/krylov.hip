@@ -52,7 +52,6 @@ __device__ __forceinline__ double lane_val(double v, int i) {
   const unsigned hi = __builtin_amdgcn_readlane((int)(u >> 32), i);
   return __longlong_as_double((long long)(((unsigned long long)hi << 32) | lo));
 }
-__device__ __forceinline__ int lane_int(int v, int i) { return __builtin_amdgcn_readlane(v, i); }
 
 // The value of the lane that a DPP control selects, `none` where there is
 // none. Reductions and scans over a wave go through these and lane reads: a

@@ -219,8 +219,8 @@ class MatrixProductState:
         """The same state with bonds widened to ``min(d^(i+1), d^(n-i-1),
         bond_dim)`` (the bond-dimension ramp of a DMRG schedule): each site
         tensor is zero-padded into the wider shape, then the state is
-        right-canonicalised (Householder LQ completes every padded bond to
-        an orthonormal basis) and normalised. Returns a new MPS."""
+        right-canonicalised (the LQ completes every padded bond to an
+        orthonormal basis) and normalised. Returns a new MPS."""
         d = self.phys_dim
         dims = [1] + _bond_dims(self.n_sites, bond_dim, d) + [1]
         out = []
