@@ -1203,16 +1203,18 @@ __global__ __launch_bounds__(256, 4) void finish_step_kernel(const double* __res
     v[i] = (VT)(w[i] * inv);
 }
 
+// nin: the partial rows that the step's cgs_step wrote, rows_blocks of the
+// count it was launched with (fewer problems may be left by now).
 template <typename VT>
-static int finish_step(VT* V, int64_t N, int J, const double* w, const double* partials, double* h3, double* sv,
-                       double* st, const TriFinish& f, double ctol, double* host_st, hipStream_t s,
+static int finish_step(VT* V, int64_t N, int J, const double* w, const double* partials, int nin, double* h3,
+                       double* sv, double* st, const TriFinish& f, double ctol, double* host_st, hipStream_t s,
                        PMap pm = kOne, int count = 1) {
   const bool rows = rows_form(N);
   // at N = 2^21 a lane writes 8 elements
   const int nb = std::min(vec_blocks(N, count), rows ? 256 : 1024);
   hipLaunchKernelGGL(finish_step_kernel<VT>, dim3(nb + 1, count), dim3(256), 0, s, w, V, N, J,
-                     rows ? partials + (size_t)2 * kRowsBlocks * kPartStride : nullptr, rows_blocks(N, count), h3, sv,
-                     st, f, ctol, host_st, pm);
+                     rows ? partials + (size_t)2 * kRowsBlocks * kPartStride : nullptr, nin, h3, sv, st, f, ctol, host_st,
+                     pm);
   TNX_LAUNCH_CHECK();
   return TNX_OK;
 }
@@ -2478,7 +2480,7 @@ static int eigsh_run(EigCtx& c, const double* v0, double* vec, double* hvec,
         // cycle, would be followed by it (no restart, not exhausted)
         const bool ahead = pipelined && J < mb && J < N && mv_now < max_mv;
         // V[j+1] = w / |w| and the projected problem
-        TNX_TRY(finish_step(V, N, J, k.w, k.partials, k.h3, k.s, k.st,
+        TNX_TRY(finish_step(V, N, J, k.w, k.partials, rows_blocks(N, 1), k.h3, k.s, k.st,
                             TriFinish{k.h1, k.h2, k.alpha, k.beta, k.T}, -1.0, ahead ? pin : nullptr, s));
         double h[4];
         if (ahead) {
@@ -2810,7 +2812,9 @@ int eigsh_heff1_b(const double* L, const double* W, const double* R, const doubl
   PinnedLease pin_lease((size_t)3 * batch);
   double* pin = pin_lease.get();
   const bool pipelined = sev.e != nullptr && pin != nullptr;
+  int prows = 0;  // partial rows of the last front
   auto front = [&](int jj) -> int {
+    prows = rows_blocks(N, cnt);
     TNX_TRY(matvec(k.V + (int64_t)jj * N, k.w, cnt));
     return cgs_step(k.V, N, jj + 1, k.w, k.partials, k.h1, k.h2, k.h3, s, pm, cnt);
   };
@@ -2836,7 +2840,7 @@ int eigsh_heff1_b(const double* L, const double* W, const double* R, const doubl
       for (int t = 0; t < steps; ++t) {
         const int jj = jc + t, JJ = jj + 1;
         TNX_TRY(front(jj));
-        TNX_TRY(finish_step(k.V, N, JJ, k.w, k.partials, k.h3, k.s, k.st,
+        TNX_TRY(finish_step(k.V, N, JJ, k.w, k.partials, prows, k.h3, k.s, k.st,
                             TriFinish{k.h1, k.h2, k.alpha, k.beta, k.T}, tol, nullptr, s, pm, cnt));
       }
       const int Jl = jc + steps;  // basis rows after the last step
@@ -2918,7 +2922,7 @@ int eigsh_heff1_b(const double* L, const double* W, const double* R, const doubl
     const int J = j + 1;
     if (!queued) TNX_TRY(front(j));
     const int mv_now = matvecs;
-    TNX_TRY(finish_step(k.V, N, J, k.w, k.partials, k.h3, k.s, k.st,
+    TNX_TRY(finish_step(k.V, N, J, k.w, k.partials, prows, k.h3, k.s, k.st,
                         TriFinish{k.h1, k.h2, k.alpha, k.beta, k.T}, -1.0, nullptr, s, pm, cnt));
     const bool ahead = pipelined && J < mb && J < N && mv_now < max_mv;
     if (ahead) {
