@@ -847,6 +847,27 @@ __device__ __forceinline__ void twisted_minors(TriLds& t, int n, double x) {
   for (; i < n; ++i) step(ra[i * dir].x, rb[i * dir].y, i);
 }
 
+// The same pivots by their own recurrence q_k = a_k - x - b_{k-1}^2 / q_{k-1},
+// {q_k, 1}, where one below `tiny` is replaced by it before the next is formed.
+// A minor that is zero, or a rounding error, leaves a finite pivot behind it
+// that belongs to a matrix within `tiny` of T. A reciprocal a row instead of
+// two products (80 cycles against 16).
+__device__ __forceinline__ void twisted_pivots(TriLds& t, int n, double x, double tiny) {
+  const int lane = threadIdx.x;
+  const bool up = lane >= 32, wr = (lane & 31) == 0;
+  const double2* ra = up ? t.row + (n - 1) : t.row;
+  const double2* rb = up ? t.row + n : t.row;
+  double2* qo = up ? t.q[1] + (n - 1) : t.q[0];
+  const int dir = up ? -1 : 1;
+  double q = 0.0;
+  for (int i = 0; i < n; ++i) {
+    const double c = i > 0 ? rb[i * dir].y * rcp_nr(q) : 0.0;
+    q = ra[i * dir].x - x - c;
+    if (!(fabs(q) >= tiny)) q = tiny;
+    if (wr) qo[i * dir] = make_double2(q, 1.0);
+  }
+}
+
 // The lowest eigenpair for n <= 64 NC (NC = 1: every Lanczos projection), by
 // one wave; row k = 64 c + lane in register c of its lane.
 //
@@ -979,70 +1000,97 @@ __device__ __forceinline__ void tridiag_lowest_wave(TriLds& t, const double* __r
   // Eigenvector: pivots q+ from above and q- from below; row r where
   // gamma = q+ + q- - (a - theta) is smallest is where the two meet, and
   // z_r = 1, z_k = -b_k / q+_k z_{k+1} above it, -b_{k-1} / q-_k z_{k-1}
-  // below.
+  // below. The pivots come from ratios of minors, which lose them where the
+  // lowest level is degenerate: a level that two uncoupled blocks share makes
+  // the minors from both ends zero, and 0 / 0 says nothing of r; blocks coupled
+  // at rounding level give two nearly singular pivots that cancel (residuals up
+  // to 1e-11 |T|). So the residual is looked at, and a vector beyond 6 eps |T|
+  // (the others stay below 5.5) is formed again from the guarded recurrence,
+  // whose residuals stay below that on such matrices too.
+  const double tiny = fmax(eps * tnorm, 1e-290);
+  double z[NC], nn = 0.0, mx = 0.0;
+  auto twisted = [&]() {
+    double up[NC], dn[NC], gam[NC], gmin = 1e308;
+#pragma unroll
+    for (int c = 0; c < NC; ++c) {
+      const int k = 64 * c + lane;
+      up[c] = dn[c] = 1.0;
+      gam[c] = 1e308;
+      if (k < n) {
+        const double2 a = t.q[0][k], b = t.q[1][k];
+        double qp = a.x / a.y, qm = b.x / b.y;
+        const double gm = fabs(qp + qm - (ar[c] - theta));
+        if (gm < 1e308) gam[c] = gm;  // not for a NaN or an infinity
+        if (!(fabs(qp) >= tiny)) qp = tiny;
+        if (!(fabs(qm) >= tiny)) qm = tiny;
+        up[c] = -bn[c] / qp;
+        dn[c] = -bl[c] / qm;
+      }
+      gmin = fmin(gmin, gam[c]);
+    }
+    gmin = wave_min(gmin);
+    int r = -1;
+#pragma unroll
+    for (int c = 0; c < NC; ++c) {
+      const unsigned long long at = __ballot(gam[c] == gmin && 64 * c + lane < n);
+      if (r < 0 && at != 0ull) r = 64 * c + __ffsll((long long)at) - 1;
+    }
+    double carry = 1.0;
+    // below r: running products downwards
+#pragma unroll
+    for (int c = 0; c < NC; ++c) {
+      const int k = 64 * c + lane;
+      double f = k > r && k < n ? dn[c] : 1.0;
+      for (int o = 1; o < 64; o <<= 1) {
+        const double v = __shfl_up(f, o, 64);
+        if (lane >= o) f *= v;
+      }
+      z[c] = f * carry;
+      if (NC > 1) carry = lane_val(z[c], 63);
+    }
+    // above r: running products upwards
+    carry = 1.0;
+#pragma unroll
+    for (int c = NC - 1; c >= 0; --c) {
+      const int k = 64 * c + lane;
+      double f = k < r ? up[c] : 1.0;
+      for (int o = 1; o < 64; o <<= 1) {
+        const double v = __shfl_down(f, o, 64);
+        if (lane + o < 64) f *= v;
+      }
+      f *= carry;
+      if (NC > 1) carry = lane_val(f, 0);
+      z[c] = k < n ? z[c] * f : 0.0;
+    }
+    nn = 0.0;
+    mx = 0.0;
+#pragma unroll
+    for (int c = 0; c < NC; ++c) {
+      nn += z[c] * z[c];
+      mx = fmax(mx, fabs(z[c]));
+    }
+    nn = wave_sum(nn);
+    mx = wave_max(mx);
+  };
   twisted_minors(t, n, theta);
   wave_lds_fence();
-  const double tiny = fmax(eps * tnorm, 1e-290);
-  double up[NC], dn[NC], gam[NC], gmin = 1e308;
+  twisted();
+  double rm = 0.0;
 #pragma unroll
   for (int c = 0; c < NC; ++c) {
-    const int k = 64 * c + lane;
-    up[c] = dn[c] = 1.0;
-    gam[c] = 1e308;
-    if (k < n) {
-      const double2 a = t.q[0][k], b = t.q[1][k];
-      double qp = a.x / a.y, qm = b.x / b.y;
-      const double gm = fabs(qp + qm - (ar[c] - theta));
-      if (gm < 1e308) gam[c] = gm;  // not for a NaN or an infinity
-      if (!(fabs(qp) >= tiny)) qp = tiny;
-      if (!(fabs(qm) >= tiny)) qm = tiny;
-      up[c] = -bn[c] / qp;
-      dn[c] = -bl[c] / qm;
-    }
-    gmin = fmin(gmin, gam[c]);
+    double zu = dpp<0x138>(z[c]), zd = dpp<0x130>(z[c]);  // wave_shr 1, wave_shl 1
+    if (c > 0 && lane == 0) zu = lane_val(z[c > 0 ? c - 1 : 0], 63);
+    if (c + 1 < NC && lane == 63) zd = lane_val(z[c + 1 < NC ? c + 1 : c], 0);
+    const double rk = fabs(fma(ar[c] - theta, z[c], fma(bl[c], zu, bn[c] * zd)));
+    rm = fmax(rm, 64 * c + lane < n ? (rk <= 1e300 ? rk : 1e308) : 0.0);  // a NaN counts
   }
-  gmin = wave_min(gmin);
-  int r = -1;
-#pragma unroll
-  for (int c = 0; c < NC; ++c) {
-    const unsigned long long at = __ballot(gam[c] == gmin && 64 * c + lane < n);
-    if (r < 0 && at != 0ull) r = 64 * c + __ffsll((long long)at) - 1;
+  rm = wave_max(rm);
+  if (!(rm <= 6.0 * eps * tnorm * sqrt(nn) && nn < 1e300)) {
+    wave_lds_fence();
+    twisted_pivots(t, n, theta, tiny);
+    wave_lds_fence();
+    twisted();
   }
-  double z[NC], carry = 1.0;
-  // below r: running products downwards
-#pragma unroll
-  for (int c = 0; c < NC; ++c) {
-    const int k = 64 * c + lane;
-    double f = k > r && k < n ? dn[c] : 1.0;
-    for (int o = 1; o < 64; o <<= 1) {
-      const double v = __shfl_up(f, o, 64);
-      if (lane >= o) f *= v;
-    }
-    z[c] = f * carry;
-    if (NC > 1) carry = lane_val(z[c], 63);
-  }
-  // above r: running products upwards
-  carry = 1.0;
-#pragma unroll
-  for (int c = NC - 1; c >= 0; --c) {
-    const int k = 64 * c + lane;
-    double f = k < r ? up[c] : 1.0;
-    for (int o = 1; o < 64; o <<= 1) {
-      const double v = __shfl_down(f, o, 64);
-      if (lane + o < 64) f *= v;
-    }
-    f *= carry;
-    if (NC > 1) carry = lane_val(f, 0);
-    z[c] = k < n ? z[c] * f : 0.0;
-  }
-  double nn = 0.0, mx = 0.0;
-#pragma unroll
-  for (int c = 0; c < NC; ++c) {
-    nn += z[c] * z[c];
-    mx = fmax(mx, fabs(z[c]));
-  }
-  nn = wave_sum(nn);
-  mx = wave_max(mx);
   // unit length; sign: largest |component| positive, the first such index on
   // ties
   double sg = 1.0 / sqrt(nn), zl = 0.0;
