@@ -2,9 +2,9 @@
 // every tensor operation in the library (H_eff matvec stages, environment
 // updates, QR trailing updates, gauge absorption): host side. FP64 and FP32
 // run the kernels of gemm_direct.h, BF16X3 (and what those do not take) the
-// LDS-tile kernels of gemm_kernel.h; this file holds that choice and, for
-// BF16X3, the split-K rule, the choice between typed and generic staging,
-// the autotuner and the tile table.
+// LDS-tile kernels of gemm_kernel.h; this file holds that choice, the split-K
+// rule of the latter and, for BF16X3, the choice between typed and generic
+// staging, the autotuner and the tile table.
 #include "gemm_direct.h"
 
 #include <cmath>
@@ -99,7 +99,7 @@ bool gemm_typed_ok(const GemmDesc& d, int kc) {
 // long K (the 32-row V^T A products of the blocked QR) otherwise run on a
 // few workgroups, each looping over all of K.
 static int split_rule(const GemmDesc& d) {
-  if (!d.splitk_ws) return 1;
+  if (!d.splitk_ws || d.gate) return 1;  // the sum of the parts has no gate
   const int64_t elems = (int64_t)d.M * d.N * d.batch;
   // about two 256x128 output tiles per CU after splitting
   const int64_t target = (int64_t)2 * 256 * 128 * 128;
@@ -237,31 +237,50 @@ bool gemm_direct_ok(const GemmDesc& d) {
          direct_operand_ok(d.tb, d.ldb, d.b_ncontig ? d.N : d.K, !d.b_ncontig);
 }
 
-// FP64 and FP32. The configuration follows a fixed rule on the shape and
-// the operand types (never on timing, addresses or strides), since the
-// K-part sum changes the rounding.
-static int run_direct(const GemmDesc& d, hipStream_t s) {
-  const GemmArgs g = args_of(d);
-  const bool f64 = d.prec == Prec::F64;
-  if (gemm_direct_ok(d)) {
-    if (f64) gemm_direct_f64(d, g, s);
-    else gemm_direct_f32(d, g, s);
-  } else {
-    if (f64) gemm_launch_f64(d, g, s);
-    else gemm_launch_f32(d, g, s);
-  }
+// The K parts of an LDS-tile launch, their length and their partial sums.
+static int set_splits(const GemmDesc& d, GemmArgs& g) {
+  const int splits = split_rule(d);
+  if (splits <= 1) return 1;
+  g.kc = ((d.K + splits - 1) / splits + 31) / 32 * 32;
+  g.partial = d.splitk_ws;
+  return ceil_div(d.K, g.kc);
+}
+
+static int sum_splits(const GemmDesc& d, const GemmArgs& g, int nsplit, hipStream_t s) {
+  if (!g.partial) return TNX_OK;
+  const int64_t MN = (int64_t)d.M * d.N;
+  const int rb = (int)std::min<int64_t>((MN + 255) / 256, 2048);
+  hipLaunchKernelGGL(splitk_reduce_kernel, dim3(rb, d.batch), dim3(256), 0, s, g.partial, nsplit, d.M, d.N, d.C,
+                     (int)d.tc, d.ldc, d.sC, d.alpha, d.beta, g.nb2, g.sC2, g.bidx);
   TNX_LAUNCH_CHECK();
   return TNX_OK;
 }
 
+// FP64 and FP32. The configuration follows a fixed rule on the shape and
+// the operand types (never on timing, addresses or strides), since the
+// K-part sum changes the rounding. What the direct kernels do not take is cut
+// by the split-K rule: matrix-vector products (N = 1) over a long K are one
+// tile, which would run on one workgroup (a step of the generalized Davidson
+// solver at chi = 256, basis rows of 131072: 64 ms against 3.1).
+static int run_direct(const GemmDesc& d, hipStream_t s) {
+  GemmArgs g = args_of(d);
+  const bool f64 = d.prec == Prec::F64;
+  if (gemm_direct_ok(d)) {
+    if (f64) gemm_direct_f64(d, g, s);
+    else gemm_direct_f32(d, g, s);
+    TNX_LAUNCH_CHECK();
+    return TNX_OK;
+  }
+  const int nsplit = set_splits(d, g);
+  if (f64) gemm_launch_f64(d, g, nsplit, s);
+  else gemm_launch_f32(d, g, nsplit, s);
+  TNX_LAUNCH_CHECK();
+  return sum_splits(d, g, nsplit, s);
+}
+
 static int run_bf16(const GemmDesc& d, hipStream_t s) {
   GemmArgs g = args_of(d);
-  const int splits = split_rule(d);
-  if (splits > 1) {
-    g.kc = ((d.K + splits - 1) / splits + 31) / 32 * 32;
-    g.partial = d.splitk_ws;
-  }
-  const int nsplit = splits > 1 ? ceil_div(d.K, g.kc) : 1;
+  const int nsplit = set_splits(d, g);
   const bool typed = gemm_typed_ok(d, g.kc);
   const TuneKey key{2, d.M, d.N, d.K, d.batch, d.a_kcontig, d.b_ncontig, (int)d.ta, (int)d.tb,
                     (int)d.tc, nsplit};
@@ -321,15 +340,7 @@ static int run_bf16(const GemmDesc& d, hipStream_t s) {
   }
   gemm_launch_bf16(ci, d, g, nsplit, typed, s);
   TNX_LAUNCH_CHECK();
-  if (g.partial) {
-    const int64_t MN = (int64_t)d.M * d.N;
-    const int rb = (int)std::min<int64_t>((MN + 255) / 256, 2048);
-    hipLaunchKernelGGL(splitk_reduce_kernel, dim3(rb, d.batch), dim3(256), 0, s, g.partial,
-                       nsplit, d.M, d.N, d.C, (int)d.tc, d.ldc, d.sC, d.alpha, d.beta,
-                       g.nb2, g.sC2, g.bidx);
-    TNX_LAUNCH_CHECK();
-  }
-  return TNX_OK;
+  return sum_splits(d, g, nsplit, s);
 }
 
 int gemm(const GemmDesc& d, hipStream_t s) {

@@ -10,8 +10,8 @@ void gemm_direct_f32(const GemmDesc& d, const GemmArgs& g, hipStream_t s) {
   return gemm_direct_run<1, float, float>(d, g, s);
 }
 
-void gemm_launch_f32(const GemmDesc& d, const GemmArgs& g, hipStream_t s) {
-  gemm_launch_index<1, void, void>(0, d, g, 1, s);
+void gemm_launch_f32(const GemmDesc& d, const GemmArgs& g, int splits, hipStream_t s) {
+  gemm_launch_index<1, void, void>(0, d, g, splits, s);
 }
 
 }  // namespace tnx

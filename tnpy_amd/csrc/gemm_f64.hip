@@ -9,8 +9,8 @@ void gemm_direct_f64(const GemmDesc& d, const GemmArgs& g, hipStream_t s) {
   return gemm_direct_run<0, double, float>(d, g, s);
 }
 
-void gemm_launch_f64(const GemmDesc& d, const GemmArgs& g, hipStream_t s) {
-  gemm_launch_index<0, void, void>(0, d, g, 1, s);
+void gemm_launch_f64(const GemmDesc& d, const GemmArgs& g, int splits, hipStream_t s) {
+  gemm_launch_index<0, void, void>(0, d, g, splits, s);
 }
 
 }  // namespace tnx

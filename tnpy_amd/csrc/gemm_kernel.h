@@ -487,8 +487,8 @@ template <> struct Cfgs<2> {
 // gemm_launch_f64 / _f32: the generic form of FP64 / FP32. gemm_launch_bf16:
 // config `ci`; `typed` selects the typed staging (the caller has checked
 // gemm_typed_ok).
-void gemm_launch_f64(const GemmDesc& d, const GemmArgs& g, hipStream_t s);
-void gemm_launch_f32(const GemmDesc& d, const GemmArgs& g, hipStream_t s);
+void gemm_launch_f64(const GemmDesc& d, const GemmArgs& g, int splits, hipStream_t s);
+void gemm_launch_f32(const GemmDesc& d, const GemmArgs& g, int splits, hipStream_t s);
 void gemm_launch_bf16(int ci, const GemmDesc& d, const GemmArgs& g, int splits, bool typed, hipStream_t s);
 
 // True when the typed staging applies: the operand types are an
