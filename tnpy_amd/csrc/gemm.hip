@@ -231,8 +231,7 @@ static bool direct_operand_ok(DT t, int64_t ld, int64_t ext, bool kcontig) {
 }
 
 bool gemm_direct_ok(const GemmDesc& d) {
-  if (d.prec == Prec::BF16X3 || (d.prec == Prec::F64 && d.ta != DT::F64)) return false;
-  return d.K >= 1 && d.lda >= 0 && d.ldb >= 0 &&
+  return d.prec != Prec::BF16X3 && d.K >= 1 && d.lda >= 0 && d.ldb >= 0 &&
          direct_operand_ok(d.ta, d.lda, d.a_kcontig ? d.K : d.M, d.a_kcontig) &&
          direct_operand_ok(d.tb, d.ldb, d.b_ncontig ? d.N : d.K, !d.b_ncontig);
 }

@@ -495,9 +495,9 @@ template <> struct DirectCfgs<1> {
                                      {1, 1, 1, 1, 4, 4, 2}, {1, 1, 2, 2, 1, 4, 2}};
 };
 
-// True where the kernel applies: an instantiated pair of operand types, a
-// pair to load along each operand's contiguous dimension, and offsets inside
-// a wave's tile within a buffer's 2 GiB range.
+// True where the kernel applies: FP64 or FP32 arithmetic, a pair to load
+// along each operand's contiguous dimension, and offsets inside a wave's tile
+// within a buffer's 2 GiB range.
 bool gemm_direct_ok(const GemmDesc& d);
 
 void gemm_direct_f64(const GemmDesc& d, const GemmArgs& g, hipStream_t s);

@@ -4,9 +4,10 @@
 namespace tnx {
 
 void gemm_direct_f64(const GemmDesc& d, const GemmArgs& g, hipStream_t s) {
-  // (F64, F64) and (F64, F32): the pairs gemm_direct_ok admits for F64
-  if (d.tb == DT::F64) return gemm_direct_run<0, double, double>(d, g, s);
-  return gemm_direct_run<0, double, float>(d, g, s);
+  if (d.ta == DT::F64 && d.tb == DT::F64) return gemm_direct_run<0, double, double>(d, g, s);
+  if (d.ta == DT::F64) return gemm_direct_run<0, double, float>(d, g, s);
+  if (d.tb == DT::F64) return gemm_direct_run<0, float, double>(d, g, s);
+  return gemm_direct_run<0, float, float>(d, g, s);
 }
 
 void gemm_launch_f64(const GemmDesc& d, const GemmArgs& g, int splits, hipStream_t s) {

@@ -4,8 +4,8 @@
 // runs the BF16X3 arithmetic, whose operands are split into two bf16 planes
 // once per tile, and the FP64 / FP32 products that gemm_direct.h (registers
 // straight from memory, faster everywhere else) does not take: operands
-// without a pair along their contiguous dimension, or mixed types it has no
-// instantiation for.
+// without a pair along their contiguous dimension, or out of its range of
+// offsets.
 //
 // One kernel template, three arithmetics:
 //   F64    : v_mfma_f64_16x16x4_f64, FP64 LDS tiles [BK][BM]
