@@ -1049,7 +1049,8 @@ size_t qr_ws_bytes(int m, int n) {
 // them with `after` already queued, and queues it again where A had to be
 // factored a second time.
 template <class After>
-static int qr_then(double* A, int m, int n, double* R, void* ws, size_t ws_bytes, hipStream_t s, After after) {
+static int qr_then(double* A, int m, int n, double* R, void* ws, size_t ws_bytes, hipStream_t s, QrUse use,
+                   After after) {
   TNX_CHECK_ARG(A && R, "qr: null pointer");
   TNX_CHECK_ARG(m >= 1 && n >= 1 && m >= n, "qr: need m >= n >= 1 (m=%d n=%d)", m, n);
   QrCfg c;
@@ -1065,9 +1066,14 @@ static int qr_then(double* A, int m, int n, double* R, void* ws, size_t ws_bytes
   char* p = (char*)(((uintptr_t)ws + 255) & ~(uintptr_t)255);
   double* save = (double*)p; p += al((size_t)m * n * 8);
   TNX_TRY(copy_f64(A, save, (int64_t)m * n, s));
-  // A thread whose last matrix took more than two passes queues all four at
-  // once (the same kind of matrix again, mostly): the results are the same.
-  static thread_local bool more = false;
+  // A thread whose last matrix of the same use took more than two passes queues
+  // all four at once: the results are the same, and a wrong guess costs a second
+  // factorisation (two queued, four wanted) or the gated launches. One use says
+  // nothing of the next: a truncation factors its matrix, the graded factor of
+  // that and an almost orthonormal basis in turn (one guess for the three: 8.15
+  // ms at n = 512, 70.7 at 2048; one each: 7.7, 68.0).
+  static thread_local bool more_of[(int)QrUse::Count] = {};
+  bool& more = more_of[(int)use];
   const int nf = wp_panels(n) * kWpFlags;
   PinnedLease pin((size_t)(nf + 1) / 2);
   StepEvent fev;
@@ -1106,8 +1112,8 @@ static int qr_then(double* A, int m, int n, double* R, void* ws, size_t ws_bytes
   return after();
 }
 
-int qr(double* A, int m, int n, double* R, void* ws, size_t ws_bytes, hipStream_t s) {
-  return qr_then(A, m, n, R, ws, ws_bytes, s, [] { return TNX_OK; });
+int qr(double* A, int m, int n, double* R, void* ws, size_t ws_bytes, hipStream_t s, QrUse use) {
+  return qr_then(A, m, n, R, ws, ws_bytes, s, use, [] { return TNX_OK; });
 }
 
 // ---- gauge moves -------------------------------------------------------------
@@ -1129,7 +1135,7 @@ int gauge_right(double* A, const double* next, double* next_out, int chil, int d
   TNX_CHECK_ARG(ws && ws_bytes >= gauge_ws_bytes(chil, d, chir), "gauge_right: workspace too small");
   char* p = (char*)(((uintptr_t)ws + 255) & ~(uintptr_t)255);
   double* R = (double*)p; p += al((size_t)n * n * 8);
-  return qr_then(A, m, n, R, p, qr_ws_bytes(m, n), s, [&]() -> int {
+  return qr_then(A, m, n, R, p, qr_ws_bytes(m, n), s, QrUse::GaugeRight, [&]() -> int {
     // next_out = R * next
     GemmDesc g{};
     g.M = n; g.N = next_cols; g.K = n; g.batch = 1;
@@ -1166,7 +1172,7 @@ int gauge_left(double* A, const double* prev, double* prev_out, int chil, int d,
     return carry();
   }
   TNX_TRY(transpose_f64(A, At, n, m, s));
-  return qr_then(At, m, n, R, p, qr_ws_bytes(m, n), s, [&]() -> int {
+  return qr_then(At, m, n, R, p, qr_ws_bytes(m, n), s, QrUse::GaugeLeft, [&]() -> int {
     TNX_TRY(transpose_f64(At, A, m, n, s));
     return carry();
   });
@@ -1225,7 +1231,7 @@ extern "C" {
 size_t tnx_qr_workspace_bytes(int m, int n) { return tnx::qr_ws_bytes(m, n); }
 
 int tnx_qr(double* A, int m, int n, double* R, void* ws, size_t ws_bytes, tnx_stream_t stream) {
-  return tnx::qr(A, m, n, R, ws, ws_bytes, (hipStream_t)stream);
+  return tnx::qr(A, m, n, R, ws, ws_bytes, (hipStream_t)stream, tnx::QrUse::Plain);
 }
 
 size_t tnx_gauge_workspace_bytes(int chil, int d, int chir) {

@@ -38,9 +38,6 @@
 
 namespace tnx {
 
-int qr(double* A, int m, int n, double* R, void* ws, size_t ws_bytes, hipStream_t s);
-size_t qr_ws_bytes(int m, int n);
-
 constexpr int kJw = 32;           // rows per Jacobi block
 constexpr int kJp = 2 * kJw;      // rows of a block pair
 constexpr int kJacMaxSweeps = 30;
@@ -548,12 +545,12 @@ struct SvdScratch {
 };
 
 static int svd_core(double* S, int a, int n, int k, double* U, double* Y, double* sv_host,
-                    int* sweeps, SvdScratch& sc, hipStream_t s) {
+                    int* sweeps, SvdScratch& sc, hipStream_t s, QrUse first) {
   // S (a x n, a >= n) = Q1 R1 ; Q1 -> S in place
-  TNX_TRY(qr(S, a, n, sc.R1, sc.qws, sc.qws_bytes, s));
+  TNX_TRY(qr(S, a, n, sc.R1, sc.qws, sc.qws_bytes, s, first));
   // R1^T = Q2 R2
   TNX_TRY(transpose_f64(sc.R1, sc.T1, n, n, s));
-  TNX_TRY(qr(sc.T1, n, n, sc.R2, sc.qws, sc.qws_bytes, s));
+  TNX_TRY(qr(sc.T1, n, n, sc.R2, sc.qws, sc.qws_bytes, s, QrUse::Graded));
   double* Xj = nullptr;
   TNX_TRY(jacobi_rows(sc.R2, n, n, sc.jws, &Xj, sweeps, s));
   // rotations and the block permutation move rows through the padded
@@ -578,7 +575,7 @@ static int svd_core(double* S, int a, int n, int k, double* U, double* Y, double
                        sc.norms, k, sc.Wt);
     TNX_LAUNCH_CHECK();
   }
-  TNX_TRY(qr(sc.Wt, n, k, sc.Rw, sc.qws, sc.qws_bytes, s));
+  TNX_TRY(qr(sc.Wt, n, k, sc.Rw, sc.qws, sc.qws_bytes, s, QrUse::Basis));
   // U = Q1 W_k  (a x k)
   GemmDesc g{};
   g.M = a; g.N = k; g.K = n; g.batch = 1;
@@ -625,14 +622,14 @@ int svd_trunc(const double* X, int a, int b, int k, double* U, double* Y, double
   sc.jws = w;
   if (a >= b) {
     TNX_HIP(hipMemcpyAsync(Qa, X, sizeof(double) * (size_t)a * b, hipMemcpyDeviceToDevice, s));
-    return svd_core(Qa, a, b, k, U, Y, sv_host, sweeps, sc, s);
+    return svd_core(Qa, a, b, k, U, Y, sv_host, sweeps, sc, s, QrUse::Matrix);
   }
   // a < b: X^T (b x a) = Q0 R0, X = R0^T Q0^T; the left vectors of X are
   // those of the square R0^T, and U^T X = (U^T R0^T) Q0^T
   TNX_TRY(transpose_f64(X, Qa, a, b, s));
-  TNX_TRY(qr(Qa, b, a, R0, sc.qws, sc.qws_bytes, s));
+  TNX_TRY(qr(Qa, b, a, R0, sc.qws, sc.qws_bytes, s, QrUse::Matrix));
   TNX_TRY(transpose_f64(R0, Sq, a, a, s));
-  TNX_TRY(svd_core(Sq, a, a, k, U, Yc, sv_host, sweeps, sc, s));
+  TNX_TRY(svd_core(Sq, a, a, k, U, Yc, sv_host, sweeps, sc, s, QrUse::Graded));
   GemmDesc g{};
   g.M = k; g.N = b; g.K = a; g.batch = 1;
   g.A = Yc; g.ta = DT::F64; g.lda = a; g.sA = 0; g.a_kcontig = true;

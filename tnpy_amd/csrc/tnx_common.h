@@ -97,6 +97,12 @@ int gemm(const GemmDesc& g, hipStream_t stream);
 void set_autotune(int on);
 void tune_clear();
 
+// QR of a row-major m x n matrix (qr.hip). What it is a step of tells how many
+// passes its panels will want (see there); the result does not depend on it.
+enum class QrUse { Plain, GaugeRight, GaugeLeft, Matrix, Graded, Basis, Count };
+int qr(double* A, int m, int n, double* R, void* ws, size_t ws_bytes, hipStream_t s, QrUse use);
+size_t qr_ws_bytes(int m, int n);
+
 // While one of these lives on a host thread, the GEMMs that thread issues
 // never enter the inline tuning mode (which allocates and synchronises):
 // they take the tile table entry or the heuristic.
