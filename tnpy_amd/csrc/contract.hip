@@ -138,6 +138,9 @@ __global__ __launch_bounds__(256) void wapply_kernel(WApply a) {
   }
 }
 
+// At most kWaColumns columns a launch, which the kernel counts in 32 bits.
+constexpr int64_t kWaColumns = ((int64_t)1 << 31) - 1;
+
 static int launch_wapply(const WApply& a, hipStream_t s) {
   const int nin = a.NX * a.NY, nout = a.NP * a.NQ;
   TNX_CHECK_ARG(nout <= 64 && nin <= 64,
@@ -145,8 +148,19 @@ static int launch_wapply(const WApply& a, hipStream_t s) {
   if (a.n_outer * a.n_inner == 0) return TNX_OK;
   TNX_CHECK_ARG(a.batch >= 1 && a.batch <= 65535, "W-apply: bad batch %d", a.batch);
   const bool pair = a.n_inner >= 2;
-  const int64_t cols = a.n_outer * (pair ? (a.n_inner + 1) / 2 : a.n_inner);
-  TNX_CHECK_ARG(cols < ((int64_t)1 << 31), "W-apply: %lld points per problem", (long long)cols);
+  const int64_t per = pair ? (a.n_inner + 1) / 2 : a.n_inner, most = std::max<int64_t>(kWaColumns / per, 1);
+  if (a.n_outer > most) {
+    const int64_t es = a.in_f32 ? 4 : 8;
+    for (int64_t o = 0; o < a.n_outer; o += most) {
+      WApply part = a;
+      part.in = (const char*)a.in + o * a.in_so * es;
+      part.out = (char*)a.out + o * a.out_so * es;
+      part.n_outer = std::min(most, a.n_outer - o);
+      TNX_TRY(launch_wapply(part, s));
+    }
+    return TNX_OK;
+  }
+  const int64_t cols = a.n_outer * per;
   // one 16-column step per wave up to the 8192 waves that the chip holds;
   // one-wave blocks while those do not reach every CU
   const int64_t steps = (cols + 15) / 16;
