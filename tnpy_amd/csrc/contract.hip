@@ -44,8 +44,9 @@ struct WApply {
 // The local map on the FP64 matrix cores: out = C in, C (outputs x inputs,
 // at most 64 x 64) in registers as the A operand, the inputs of 32 points as
 // the B operand. A matrix of D d rows per point is far below the matrix
-// cores' rate, so the kernel is left bound by HBM (each value read and
-// written once) or, at small bonds, by one round of loads. The form before
+// cores' rate, so the kernel is left bound by HBM (each value written once and
+// read once per 16 outputs, a grid slice each: one reading at D d <= 16, four
+// at D d = 50) or, at small bonds, by one round of loads. The form before
 // (one point per thread, C in LDS, D d dot products of D d terms each on the
 // VALU) measured 51 us at chi = 1024, D = 5 (168 MB), 12 us at chi = 32 and
 // 137 us at chi = 200 with D = 25; this one 27 (6.1 TB/s), 3.9 and 20 us.
@@ -201,9 +202,10 @@ static bool valid_dims(int chil, int Dl, int Dr, int d, int chir) {
 // Element size of the intermediates for a given precision.
 static size_t inter_bytes(int prec) { return prec == TNX_F64 ? 8 : 4; }
 
-// Workspace: T1, T2, and FP64 split-K partials for the last GEMM (its
-// output, chil x d*chir, has few tiles at chil = chir and K = chil*Dl is
-// long; the split rule in gemm.hip decides how many are used).
+// Workspace: T1, T2, and FP64 split-K partials for the last GEMM in BF16X3
+// (its output, chil x d*chir, has few tiles at chil = chir and K = chil*Dl is
+// long; the split rule in gemm.hip decides how many are used; FP64 and FP32
+// sum parts of K inside a workgroup, but for one-column outputs):
 // partial sums of up to 4 K-splits of an output of out_elems doubles
 static size_t splitk_bytes(int64_t out_elems) { return (size_t)out_elems * 4 * 8; }
 

@@ -2297,7 +2297,7 @@ static int gd_correction(EigCtx& c, const float* V32, int J32, int keep, int m, 
   int J = kk;
   while (true) {
     // lowest Ritz pair of G (J x J): Householder tridiagonalisation,
-    // multisection + inverse iteration, back-transform into k.s
+    // multisection + twisted factorisation, back-transform into k.s
     hipLaunchKernelGGL(gd_compact_kernel, dim3(1), dim3(256), 0, s, G, J, A);
     TNX_LAUNCH_CHECK();
     if (J == 1) {
@@ -2503,12 +2503,13 @@ static int eigsh_run(EigCtx& c, const double* v0, double* vec, double* hvec,
       auto front = [&](int jj) -> int {
         if constexpr (f32) {
           if (c.L32) {
-            // FP32 basis row and FP32 environments: the matvec's GEMMs stage
-            // both operands with 16-byte loads of floats
+            // FP32 basis row and FP32 environments
             TNX_TRY(apply_h(c, V + (int64_t)jj * N, 1, k.w, cprec));
           } else {
             // FP64 environments: widen V[jj] into k.y (free until the
-            // cycle's Ritz vector is formed) for 16-byte FP64 tile loads
+            // cycle's Ritz vector is formed), so both operands have one type
+            // (the BF16X3 tile table's shapes do; the FP32 products take any
+            // pair and round the widened values back to the same floats)
             hipLaunchKernelGGL(to_f64_kernel, dim3(nb), dim3(256), 0, s, V + (int64_t)jj * N, k.y, N);
             TNX_LAUNCH_CHECK();
             TNX_TRY(apply_h(c, k.y, 0, k.w, cprec));

@@ -303,7 +303,7 @@ static size_t householder_ws_bytes(int m, int n) {
   size_t b = al((size_t)m * n * 8);                 // Vall
   b += al((size_t)np * c.nb * c.nb * 8);            // T factors
   b += 2 * al((size_t)c.nb * n * 8);                // W, W2
-  b += al((size_t)32 * c.nb * n * 8);               // split-K partials
+  b += al((size_t)32 * c.nb * 8);                   // split-K partials of one-column products
   b += al((size_t)n * 8);                           // R diagonal signs
   return b + 256;
 }
@@ -342,9 +342,9 @@ static int qr_householder(double* A, int m, int n, double* R, void* ws, hipStrea
   double* Tall = (double*)p; p += al((size_t)np * NB * NB * 8);
   double* Wb = (double*)p; p += al((size_t)NB * n * 8);
   double* W2 = (double*)p; p += al((size_t)NB * n * 8);
-  double* part = (double*)p; p += al((size_t)32 * NB * n * 8);
+  double* part = (double*)p; p += al((size_t)32 * NB * 8);
   double* sg = (double*)p;
-  const size_t part_bytes = al((size_t)32 * NB * n * 8);
+  const size_t part_bytes = al((size_t)32 * NB * 8);
 
   // ---- factorisation
   for (int pi = 0; pi < np; ++pi) {

@@ -410,7 +410,7 @@ static size_t jacobi_ws_bytes(int p, int q) {
   const int npair = B / 2;
   size_t b = 2 * al((size_t)B * kJw * q * 8);       // X, Y
   b += 2 * al((size_t)npair * kJp * kJp * 8);       // G, Z
-  b += al((size_t)8 * npair * kJp * kJp * 8);       // split-K partials of the Gram GEMM
+  b += al((size_t)kFloorBlocks * 8);                // partial sums of the floor
   b += al((size_t)B * 4) + al(64);                  // perm, off bits + floor
   return b + 256;
 }
@@ -428,7 +428,7 @@ static int jacobi_rows(const double* X0, int p, int q, void* ws, double** Xout, 
   double* Y = (double*)w; w += al((size_t)rows * q * 8);
   double* G = (double*)w; w += al((size_t)npair * kJp * kJp * 8);
   double* Z = (double*)w; w += al((size_t)npair * kJp * kJp * 8);
-  double* part = (double*)w; w += al((size_t)8 * npair * kJp * kJp * 8);
+  double* part = (double*)w; w += al((size_t)kFloorBlocks * 8);
   int* perm = (int*)w; w += al((size_t)B * 4);
   unsigned long long* off_bits = (unsigned long long*)w;
   double* floor2 = (double*)(w + 8);
@@ -473,7 +473,6 @@ static int jacobi_rows(const double* X0, int p, int q, void* ws, double** Xout, 
       g.B = X; g.tb = DT::F64; g.ldb = q; g.sB = pq; g.b_ncontig = false;
       g.C = G; g.tc = DT::F64; g.ldc = kJp; g.sC = (int64_t)kJp * kJp;
       g.alpha = 1.0; g.beta = 0.0; g.prec = Prec::F64;
-      g.splitk_ws = part; g.splitk_ws_bytes = (size_t)8 * npair * kJp * kJp * 8;
       TNX_TRY(gemm(g, s));
       // a block's own pairs once per sweep, in its first round
       if (r == 0)

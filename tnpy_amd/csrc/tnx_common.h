@@ -77,8 +77,9 @@ struct GemmDesc {
   void* C;       DT tc; int64_t ldc; int64_t sC;
   double alpha, beta;
   Prec prec;
-  // Optional FP64 scratch for split-K partial sums (used when the output
-  // has few tiles and K is long); null disables splitting.
+  // Optional FP64 scratch for split-K partial sums (used by the LDS-tile
+  // kernels when the output has few tiles and K is long); null disables
+  // splitting.
   double* splitk_ws = nullptr;
   size_t splitk_ws_bytes = 0;
   // Optional second batch level: batch index b = b1 * nb2 + b2 addresses
