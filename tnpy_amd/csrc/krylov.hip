@@ -1085,7 +1085,8 @@ __device__ __forceinline__ void tridiag_lowest_wave(TriLds& t, const double* __r
     rm = fmax(rm, 64 * c + lane < n ? (rk <= 1e300 ? rk : 1e308) : 0.0);  // a NaN counts
   }
   rm = wave_max(rm);
-  if (!(rm <= 6.0 * eps * tnorm * sqrt(nn) && nn < 1e300)) {
+  const double lim = 6.0 * eps * tnorm;
+  if (!(rm * rm <= lim * lim * nn && nn < 1e200)) {
     wave_lds_fence();
     twisted_pivots(t, n, theta, tiny);
     wave_lds_fence();
